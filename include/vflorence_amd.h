@@ -473,6 +473,24 @@ int vfl_layer_norm_apply(const void *v, int64_t v_stride, const float *v_stats,
                          const void *gamma, const void *beta, float eps, void *out,
                          int64_t out_stride, int64_t rows, int dim, int dtype, void *stream);
 
+/*
+ * Encoder self-attention of packed prompts (scaled_dot_product_attention per prompt in the
+ * reference's encoder, vflorence/models/bart.py; no vllm_cpu_attn counterpart):
+ * out[r][h] = softmax(scale * q[r][h] K[h]^T) V[h] over the tokens of r's own prompt.
+ * segments (HOST memory, read during the call): num_segments triples (start, count,
+ * length), each naming `count` prompts of `length` tokens stored back to back from token
+ * `start` on, within the num_tokens rows; rows that no segment names are neither read nor
+ * written.  q, k and v: rows of num_heads x head_dim elements at one row stride (the
+ * thirds of a fused q|k|v projection), 16-byte aligned, the stride a multiple of 8; out
+ * 8-byte aligned, its stride a multiple of 4.  bf16 and fp16, head_dim 64 (else
+ * VFL_E_UNSUPPORTED), scale > 0.  Scores, softmax and sums in fp32, the weights rounded to
+ * the element type for the second product.  One launch per 128 segments.
+ */
+int vfl_encoder_attention(const void *q, const void *k, const void *v, int64_t stride, void *out,
+                          int64_t out_stride, int64_t num_tokens, const int64_t *segments,
+                          int64_t num_segments, int num_heads, int head_dim, float scale,
+                          int dtype, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,78 @@
+"""Packed encoder attention (vfl_encoder_attention) against fp64 softmax attention."""
+
+import pytest
+import torch
+
+from vflorence_amd import hip_attn
+from vflorence_amd.layers.bart import BartEncoderSelfAttention
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(qkv, segments, heads):
+    """(attention, attention of |v|) per prompt in fp64; rows outside every run are zero."""
+    n, d = qkv.shape[0], qkv.shape[1] // 3
+    out = torch.zeros(2, n, d, dtype=torch.float64, device=qkv.device)
+    for start, count, length in segments:
+        for at in range(start, start + count * length, max(length, 1)):
+            q, k, v = (t.double().view(length, heads, 64).transpose(0, 1)
+                       for t in qkv[at:at + length].chunk(3, dim=-1))
+            p = torch.softmax(q @ k.transpose(1, 2).contiguous() / 8, -1)
+            for i, x in enumerate((v, v.abs())):
+                out[i, at:at + length] = (p @ x.contiguous()).transpose(0, 1).reshape(length, d)
+    return out
+
+
+def check(out, qkv, segments, heads):
+    ref, size = reference(qkv, segments, heads)
+    # each weight and each output is rounded once, by at most u = 2^-p for p significant
+    # bits (8 in bf16, 11 in fp16); fp16 weights below 2^-14 of the
+    # largest lose at most 2^-25 each; 2e-5 for the fp32 scores and sums
+    u = 2.0**-8 if qkv.dtype == torch.bfloat16 else 2.0**-11
+    tiny = max(n for _, _, n in segments) * 2.0**-25 * float(qkv.abs().max())
+    bound = 1.05 * u * (size + ref.abs()) + 2e-5 * size + tiny + 1e-6
+    err = (out.double() - ref).abs()
+    assert bool((err <= bound).all()), float((err / bound).max())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("heads, runs", [
+    (1, [(1, 1)]),                                   # one key
+    (3, [(2, 31), (1, 32), (1, 33), (3, 64)]),       # edges of the query and key tiles
+    (12, [(1, 590)]),                                # two key groups
+    (1, [(1, 65)]), (2, [(1, 200)]),                 # as many key groups as key tiles; four
+    (16, [(4, 129), (1, 127), (2, 128)]),            # two key groups
+    (16, [(8, 1000), (0, 7), (5, 65), (3, 0)]),      # one key group; empty runs
+    (2, [(1, 1 + 3 * i) for i in range(150)]),       # more runs than one launch holds
+])
+def test_packed_prompts(dtype, heads, runs):
+    g = torch.Generator(device="cuda").manual_seed(heads)
+    segments, at = [], 3  # three rows before the first run
+    for count, length in runs:
+        segments.append((at, count, length))
+        at += count * length
+    # strided rows; rows that no run names hold NaN, which nothing may read
+    qkv = torch.randn(at + 5, 3 * heads * 64 + 8, generator=g, device="cuda").to(dtype)
+    qkv = qkv[:, :3 * heads * 64].mul_(2)
+    qkv[:3], qkv[at:] = float("nan"), float("nan")
+    out = torch.full((at + 5, heads * 64), 7.0, dtype=dtype, device="cuda")
+    assert hip_attn.encoder_attention_fits(qkv, out, heads, 0.125)
+    hip_attn.encoder_attention(qkv, segments, out, heads, 0.125)
+    assert bool((out[:3] == 7).all()) and bool((out[at:] == 7).all())
+    check(out[3:at], qkv[3:at], [(s - 3, c, n) for s, c, n in segments], heads)
+
+
+def test_layer_forms():
+    """The layer's three callers agree, and a call with a gradient keeps torch's path."""
+    torch.manual_seed(0)
+    layer = BartEncoderSelfAttention(128, 2).cuda().to(torch.bfloat16)
+    x = torch.randn(3, 45, 128, device="cuda").to(torch.bfloat16)
+    with torch.no_grad():
+        a = layer(x)
+        b = layer(x.view(-1, 128), [(0, 3, 45)]).view_as(a)
+    assert torch.equal(a, b)
+    c = layer(x)
+    c.float().sum().backward()
+    assert layer.qkv_proj.weight.grad is not None
+    c = c.detach()
+    assert float((a - c).float().norm() / c.float().norm()) < 1e-2  # two bf16 roundings

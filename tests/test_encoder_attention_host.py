@@ -1,0 +1,35 @@
+"""vfl_encoder_attention's argument checks and the calls that keep torch's path (CPU)."""
+
+import ctypes
+
+import pytest
+import torch
+
+from vflorence_amd import hip_attn
+from vflorence_amd._lib import lib
+from vflorence_amd.layers.bart import _runs_fit
+
+
+def call(segments=((0, 1, 4),), heads=2, dim=64, stride=384, scale=0.125, dtype=1, tokens=4,
+         base=1 << 20, out=1 << 21):
+    flat = [x for s in segments for x in s]
+    return lib.vfl_encoder_attention(base, base + 256, base + 512, stride, out, 128, tokens,
+                                     (ctypes.c_int64 * len(flat))(*flat), len(segments), heads,
+                                     dim, scale, dtype, None)
+
+
+@pytest.mark.parametrize("bad", [
+    dict(dtype=0), dict(dim=128), dict(heads=0), dict(scale=0.0), dict(stride=100),
+    dict(stride=388), dict(base=8), dict(out=(1 << 21) + 4),
+    dict(segments=((0, 1, 5),)), dict(segments=((1, 1, 4),)), dict(segments=((-1, 1, 2),)),
+    dict(segments=((0, 2, 3),)), dict(segments=((0, 1 << 62, 4),)), dict(segments=((0, -1, 2),)),
+])
+def test_refused_calls(bad):
+    assert call(**bad) < 0 and lib.vfl_last_error()
+
+
+def test_runs_and_plain_calls():
+    assert _runs_fit([(0, 2, 3), (6, 0, 5), (6, 1, 4)], 10)
+    assert not _runs_fit([(0, 2, 3)], 5) and not _runs_fit([(3, 1, 2), (0, 1, 2)], 9)
+    assert not hip_attn.encoder_attention_fits(torch.zeros(4, 384, dtype=torch.bfloat16), None, 2,
+                                               0.125)

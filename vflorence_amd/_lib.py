@@ -22,6 +22,7 @@ VFL_OK = 0
 EXPORTED_SYMBOLS = (
     "vfl_last_error",
     "vfl_version",
+    "vfl_encoder_attention",
     "vfl_get_isa",
     "vfl_reshape_and_cache",
     "vfl_get_scheduler_metadata",
@@ -135,6 +136,10 @@ _SIGNATURES = {
     "vfl_linear_norm": (
         ctypes.c_int,
         [_vp, _i64, _vp, _f32, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _i32, _i32, _vp],
+    ),
+    "vfl_encoder_attention": (
+        ctypes.c_int,
+        [_vp, _vp, _vp, _i64, _vp, _i64, _i64, _vp, _i64, _i32, _i32, _f32, _i32, _vp],
     ),
     "vfl_layer_norm_apply": (
         ctypes.c_int,

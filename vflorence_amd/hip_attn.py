@@ -679,6 +679,53 @@ def self_attention_with_kv_write(
     )
 
 
+ENCODER_HEAD_DIM = 64  # head size of the packed encoder attention kernel
+
+
+def encoder_attention_fits(qkv: torch.Tensor, out: torch.Tensor | None, num_heads: int,
+                           scale: float) -> bool:
+    """Whether ``encoder_attention`` serves these ``[tokens, 3 d]`` projections: 16-bit GPU
+    tensors of 64-wide heads whose rows are aligned for its loads, in a plain eager call
+    (nothing to differentiate, trace, batch or dispatch elsewhere)."""
+    if not (type(qkv) is torch.Tensor and qkv.is_cuda
+            and qkv.dtype in (torch.bfloat16, torch.float16)
+            and qkv.dim() == 2 and qkv.shape[1] == 3 * num_heads * ENCODER_HEAD_DIM
+            and scale > 0):
+        return False
+    if (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
+            or torch._C._len_torch_dispatch_stack()
+            or torch._C._functorch.maybe_current_level() is not None
+            or torch.autograd.forward_ad._current_level >= 0
+            or (qkv.requires_grad and torch.is_grad_enabled())):
+        return False
+    if qkv.stride(1) != 1 or qkv.stride(0) % 8 or qkv.data_ptr() % 16:
+        return False
+    return out is None or (type(out) is torch.Tensor and out.device == qkv.device
+                           and out.dtype == qkv.dtype and out.dim() == 2
+                           and not out.requires_grad
+                           and out.shape[1] == num_heads * ENCODER_HEAD_DIM
+                           and out.stride(1) == 1 and out.stride(0) % 4 == 0
+                           and out.stride(0) >= out.shape[1] and out.data_ptr() % 8 == 0)
+
+
+def encoder_attention(qkv: torch.Tensor, segments, out: torch.Tensor, num_heads: int,
+                      scale: float) -> None:
+    """Self-attention of packed prompts (``vfl_encoder_attention``): ``qkv`` ``[tokens, 3 d]``
+    holds each token's q, k and v, ``segments`` lists ``(start, count, length)`` runs of
+    equal-length prompts, and the rows they name of ``out`` ``[tokens, d]`` are written.
+    For calls that ``encoder_attention_fits`` accepts."""
+    tokens = min(qkv.shape[0], out.shape[0])
+    if tokens == 0:
+        return
+    flat = [int(x) for run in segments for x in run]
+    triples = (ctypes.c_int64 * len(flat))(*flat)
+    d, base, size = num_heads * ENCODER_HEAD_DIM, qkv.data_ptr(), qkv.element_size()
+    check(lib.vfl_encoder_attention(
+        base, base + d * size, base + 2 * d * size, qkv.stride(0), out.data_ptr(), out.stride(0),
+        tokens, triples, len(flat) // 3, num_heads, ENCODER_HEAD_DIM, float(scale),
+        _dtype_code(qkv.dtype), _stream(qkv.device)))
+
+
 def cache_pointer_table(caches: list[torch.Tensor]) -> torch.Tensor:
     """Device int64 tensor of cache base addresses, the ``caches`` argument of copy_blocks."""
     if not caches:

@@ -11,8 +11,9 @@ the encoder K/V that ``ModelRunner._encode`` paged once per request.  ``scaling`
 Module and parameter names follow the transformers BART checkpoint layout
 (``model.encoder.layers.N.self_attn...``, ``lm_head``, ``final_logits_bias``) so a
 checkpoint's state dict loads after its q/k/v projections are concatenated
-(``fuse_projections``).  The encoder runs dense attention with torch's SDPA on the
-GPU: it is outside the decode path.  One decode step is ``forward(input_ids,
+(``fuse_projections``).  The encoder's attention is one launch over all packed prompts
+for 16-bit GPU tensors of 64-wide heads (``hip_attn.encoder_attention``), torch's SDPA
+per run of equal-length prompts otherwise.  One decode step is ``forward(input_ids,
 positions)`` over one token per running sequence.
 """
 
@@ -25,6 +26,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
+from .. import hip_attn
 from ..decoder_ops import LINEAR_MAX_IN, LINEAR_MAX_OUT, LINEAR_MAX_ROWS
 from .attention import decoder_cross_attention, decoder_self_attention
 
@@ -254,6 +256,17 @@ class _Heads(nn.Module):
         self.scaling = self.head_dim**-0.5
 
 
+def _runs_fit(segments, rows: int) -> bool:
+    """Whether the ``(start, count, length)`` runs lie within ``rows`` rows and do not
+    overlap in order (what the packed attention kernel takes; SDPA judges the rest)."""
+    at = 0
+    for start, count, length in segments:
+        if start < at or count < 0 or length < 0:
+            return False
+        at = start + count * length
+    return at <= rows
+
+
 class BartEncoderSelfAttention(_Heads):
     fused_projections = {"qkv_proj": ("q_proj", "k_proj", "v_proj")}
 
@@ -270,8 +283,14 @@ class BartEncoderSelfAttention(_Heads):
         of equal-length prompts."""
         if segments is None:
             b, s, _ = x.shape
+            qkv = self.qkv_proj(x)
+            rows = qkv.reshape(b * s, 3 * self.embed_dim)
+            if hip_attn.encoder_attention_fits(rows, None, self.num_heads, self.scaling):
+                out = rows.new_empty(b * s, self.embed_dim)
+                hip_attn.encoder_attention(rows, ((0, b, s),), out, self.num_heads, self.scaling)
+                return out.view(b, s, self.embed_dim)
             q, k, v = (t.view(b, s, self.num_heads, self.head_dim).transpose(1, 2)
-                       for t in self.qkv_proj(x).chunk(3, dim=-1))
+                       for t in qkv.chunk(3, dim=-1))
             out = F.scaled_dot_product_attention(q, k, v, scale=self.scaling)
             return out.transpose(1, 2).reshape(b, s, self.embed_dim)
         out = x.new_empty(x.shape[0], self.embed_dim)
@@ -281,7 +300,12 @@ class BartEncoderSelfAttention(_Heads):
     def attend(self, qkv: torch.Tensor, segments, out: torch.Tensor) -> None:
         """Attention of each run of equal-length prompts over the packed projections
         ``qkv`` [>= T, 3 d], written to rows ``start .. start + count * length`` of
-        ``out``; other rows are left as they are."""
+        ``out``; other rows are left as they are.  One launch for all runs where the
+        packed kernel serves the call (hip_attn.encoder_attention_fits), else SDPA per run."""
+        if (hip_attn.encoder_attention_fits(qkv, out, self.num_heads, self.scaling)
+                and _runs_fit(segments, min(qkv.shape[0], out.shape[0]))):
+            hip_attn.encoder_attention(qkv, segments, out, self.num_heads, self.scaling)
+            return
         for start, count, length in segments:
             end = start + count * length
             q, k, v = (t.view(count, length, self.num_heads, self.head_dim).transpose(1, 2)
