@@ -281,8 +281,8 @@ int vfl_attention_with_kv_cache(const void *query, int64_t query_stride_token,
  * table, or a slot that no row of this call attends to; and the block holding a
  * row's new token is read by no other row.  Then the result -- cache contents and
  * out -- equals reshape_and_cache followed by attention_with_kv_cache.  Callers that
- * cannot vouch for it use those two entry points.  fp32 caches, and head sizes other
- * than 64 and 128, run the two steps.
+ * cannot vouch for it use those two entry points.  Head sizes other than 64 and 128
+ * run the two steps.
  *
  * key / value: [num_rows][num_heads][head_dim] with token / head strides in
  * elements (the strided views of a fused qkv projection).  Other arguments as for

@@ -50,17 +50,21 @@ inline bool head_dim_native(int d) { return d == 64 || d == 128; }
 
 // fp32 caches: VALU kernel over the logical V layout, G query rows per group; pool
 // blocks of 16 << SHIFT tokens.
-template <int D, int G, int NW, int SHIFT = 0>
+template <int D, int G, int NW, int SHIFT = 0, bool FUSE = false>
 int launch_valu(const AttnArgs &a) {
   constexpr int DT = VFL_FLOAT32;
   using T = typename Elem<DT>::T;
   constexpr int BS = 16;
   const dim3 grid((unsigned)xcd_grid(a.num_groups, a.H));
-  paged_decode_kernel<DT, D, BS, G, NW, stage_blocks<DT, D, G>(), stage_pipeline<G>(), SHIFT>
+  const ValuKvWrite<DT> kvw = {(const T *)a.kvw.k, a.kvw.k_st, a.kvw.k_sh,
+                               (const T *)a.kvw.v, a.kvw.v_st, a.kvw.v_sh,
+                               a.kvw.slots,        (T *)a.kc,  (T *)a.vc};
+  paged_decode_kernel<DT, D, BS, G, NW, stage_blocks<DT, D, G>(), stage_pipeline<G>(), SHIFT,
+                      FUSE>
       <<<grid, dim3(NW * 64), 0, a.stream>>>(
       (const T *)a.q, a.q_st, a.q_sh, (const T *)a.kc, (const T *)a.vc, (T *)a.out, a.seq_lens,
       a.bt, a.bt_stride, a.max_blocks, a.group_start, a.group_order, a.num_rows, a.num_groups,
-      a.H, a.num_blocks, a.scale_log2);
+      a.H, a.num_blocks, a.scale_log2, a.desc, a.desc_stride, kvw);
   return launch_status("attention_with_kv_cache");
 }
 

@@ -174,18 +174,37 @@ template <int DT> __device__ __forceinline__ typename Elem<DT>::T to_elem(float 
     return (typename Elem<DT>::T)f32_to_f16(v);
 }
 
+// The self-attention op's new tokens and the pools they are written to (KvWrite of
+// decode_mfma.h for this kernel's element type).
+template <int DT> struct ValuKvWrite {
+  using T = typename Elem<DT>::T;
+  const T *k;
+  int64_t k_st, k_sh;
+  const T *v;
+  int64_t v_st, v_sh;
+  const int64_t *slots;
+  T *kc, *vc;
+};
+
 // SHIFT: pool blocks hold BS << SHIFT tokens (0, or 1 for the reference's 32-token
 // blocks); the kernel walks BS-token parts of them.
-template <int DT, int D, int BS, int G, int NW, int U, bool PIPE, int SHIFT>
+// FUSE (one row per workgroup): also writes the row's new token at its slot, under the
+// fused write's contract (see paged_decode_mfma_kernel, and desc there).  Where the slot is the row's last
+// position, the wave that reads that block puts the token into its registers and stores
+// it; a slot elsewhere is written by wave 0.  With a separate scatter launch the 64 rows
+// x 72 tokens of a layer took 4.8 + 9.4 us, fused 10.0.
+template <int DT, int D, int BS, int G, int NW, int U, bool PIPE, int SHIFT, bool FUSE>
 __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(
     const typename Elem<DT>::T *__restrict__ q, int64_t q_st, int64_t q_sh,
     const typename Elem<DT>::T *__restrict__ kc, const typename Elem<DT>::T *__restrict__ vc,
     typename Elem<DT>::T *__restrict__ out, const int32_t *__restrict__ seq_lens,
     const int32_t *__restrict__ bt, int64_t bt_stride, int max_blocks,
     const int32_t *__restrict__ group_start, const int32_t *__restrict__ group_order,
-    int64_t num_rows, int64_t num_groups, int H, int64_t num_blocks, float scale_log2) {
+    int64_t num_rows, int64_t num_groups, int H, int64_t num_blocks, float scale_log2,
+    const int32_t *__restrict__ desc, int64_t desc_stride, ValuKvWrite<DT> kvw) {
   using Lay = ValuLayout<DT, D>;
   constexpr int bs_shift = SHIFT;
+  static_assert(!FUSE || (G == 1 && SHIFT == 0 && !PIPE), "the fused write is one row's");
   constexpr int VEC = Lay::VEC, CPL = Lay::CPL, LPT = Lay::LPT, TPL = Lay::TPL;
   constexpr int NLD = BS / TPL;  // loads per block per head and chunk slot
   static_assert(64 % LPT == 0 && BS % TPL == 0, "unsupported tile");
@@ -200,25 +219,57 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(
   int64_t pos;
   int h;
   xcd_position(blockIdx.x, (unsigned)H, pos, h);
-  if (pos >= num_groups) return;  // workgroup-uniform
-  int g = (int)pos;
-  if (group_order) g = group_order[g];
   // Workgroup-uniform exits only (before any barrier).
-  if (g < 0 || g >= num_groups || h >= H) return;
-  int row0 = g, nrows = 1;
-  if (group_start) {
-    row0 = group_start[g];
-    nrows = min(group_start[g + 1] - row0, G);
+  if (pos >= num_groups || h >= H) return;
+  int row0, nrows = 1, L;
+  WaveBlockIds ids;
+  const bool described = G > 1 && SHIFT == 0 && desc != nullptr;
+  if (described) {
+    const int32_t *rec = desc + pos * desc_stride;
+    const int4 hdr = *reinterpret_cast<const int4 *>(rec);
+    ids.prefetch(rec + 4, max_blocks);
+    row0 = hdr.x;
+    nrows = min(hdr.y, G);
+    L = hdr.z;
+    if (row0 < 0 || row0 >= num_rows) return;
+  } else {
+    int g = (int)pos;
+    if (group_order) g = group_order[g];
+    if (g < 0 || g >= num_groups) return;
+    row0 = g;
+    if (group_start) {
+      row0 = group_start[g];
+      nrows = min(group_start[g + 1] - row0, G);
+    }
+    if (row0 < 0 || row0 >= num_rows) return;
+    L = seq_lens[row0];
   }
-  if (row0 < 0 || row0 >= num_rows) return;
   nrows = (int)min((int64_t)nrows, num_rows - row0);
   if (nrows <= 0) return;
-  const int L = seq_lens[row0];
   int nblk = L > 0 ? (L + BS - 1) / BS : 0;  // BS-token chunks
   nblk = min(nblk, max_blocks << bs_shift);
   const int Lc = min(L, nblk * BS);
   const int tok = lane / LPT;
   const int c = lane % LPT;
+
+  int last = -1, t_new = 0;  // the block and token this row's new K/V substitute
+  int64_t wslot = -1;
+  if constexpr (FUSE) {
+    wslot = kvw.slots[row0];
+    if (wslot >= num_blocks * BS) wslot = -1;
+    if (wslot >= 0 && L >= 1 && (L - 1) / BS < nblk) {
+      t_new = (L - 1) % BS;
+      const int64_t lid = bt[(int64_t)row0 * bt_stride + (L - 1) / BS];
+      if (lid * BS + t_new == wslot) last = (L - 1) / BS;
+    }
+    if (wslot >= 0 && last < 0 && wave == 0) {
+      const int64_t at = ((wslot / BS * H + h) * BS + wslot % BS) * D;
+      for (int d = lane; d < D; d += 64) {
+        kvw.kc[at + d] = kvw.k[row0 * kvw.k_st + h * kvw.k_sh + d];
+        kvw.vc[at + d] = kvw.v[row0 * kvw.v_st + h * kvw.v_sh + d];
+      }
+    }
+  }
 
   if (nblk == 0) {
     for (int i = threadIdx.x; i < nrows * D; i += NW * 64) {
@@ -253,8 +304,9 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(
     for (int d = 0; d < CPL * VEC; ++d) acc[gi][d] = 0.f;
   }
 
-  WaveBlockIds ids;
-  if constexpr (SHIFT == 0)
+  if (described)
+    ids.limit(b1);
+  else if constexpr (SHIFT == 0)
     ids.init(bt + (int64_t)row0 * bt_stride, b0, b1);
   else
     ids.init(bt + (int64_t)row0 * bt_stride, b0 >> SHIFT,
@@ -266,7 +318,23 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(
   // of stage s+1 are issued before stage s is consumed (two register stages live),
   // so each wave keeps K/V in flight while it computes; without it, latency is hidden
   // by the other waves the smaller register footprint lets the CU hold.
-  const int bfull = max(b0, min(b1, Lc / BS));
+  int bfull = max(b0, min(b1, Lc / BS));
+  const bool own_last = FUSE && b0 <= last && last < b1;
+  uint4 newk[CPL], newv[CPL];
+  if constexpr (FUSE) {  // the new token's block goes through the one-block loop below
+    if (own_last) {
+      bfull = max(b0, min(bfull, last));
+#pragma unroll
+      for (int s = 0; s < CPL; ++s) {
+        const int ch = Lay::chunk(c, s);
+        newk[s] = newv[s] = make_uint4(0, 0, 0, 0);
+        if (ch >= 0) {
+          newk[s] = load16_unaligned<DT>(kvw.k + row0 * kvw.k_st + h * kvw.k_sh + ch * VEC);
+          newv[s] = load16_unaligned<DT>(kvw.v + row0 * kvw.v_st + h * kvw.v_sh + ch * VEC);
+        }
+      }
+    }
+  }
   const int stages = (bfull - b0) / U;
   int b = b0;
   constexpr int SLOTS = U * NLD * CPL;
@@ -305,6 +373,24 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(
     bool ok[1];
     load_stage<DT, D, BS, 1, SHIFT>(kc, vc, ids, b, block_elems, lane_off, c, num_blocks, kr, vr,
                                     ok);
+    if constexpr (FUSE) {
+      if (own_last && b == last) {
+#pragma unroll
+        for (int i = 0; i < NLD; ++i) {
+          if (i * TPL + tok != t_new) continue;
+#pragma unroll
+          for (int s = 0; s < CPL; ++s) {
+            const int ch = Lay::chunk(c, s);
+            if (ch < 0) continue;
+            kr[i * CPL + s] = newk[s];
+            vr[i * CPL + s] = newv[s];
+            const int64_t at = ((wslot / BS * H + h) * BS + t_new) * D + ch * VEC;
+            *reinterpret_cast<uint4 *>(kvw.kc + at) = newk[s];
+            *reinterpret_cast<uint4 *>(kvw.vc + at) = newv[s];
+          }
+        }
+      }
+    }
     bool valid[NLD];
 #pragma unroll
     for (int i = 0; i < NLD; ++i) valid[i] = ok[0] && (b * BS + i * TPL + tok) < Lc;

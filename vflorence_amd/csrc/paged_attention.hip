@@ -94,8 +94,21 @@ static int mfma_waves(const AttnArgs &a, int nw) {
   }
 }
 
+// fp32 caches, one row per workgroup, with the KV write.
+template <int D>
+static int valu_fused(const AttnArgs &a, int nw) {
+  switch (nw) {
+    case 1: return launch_valu<D, 1, 1, 0, true>(a);
+    case 2: return launch_valu<D, 1, 2, 0, true>(a);
+    case 4: return launch_valu<D, 1, 4, 0, true>(a);
+    default: return launch_valu<D, 1, 8, 0, true>(a);
+  }
+}
+
 static int dispatch(const AttnArgs &a, int dtype, int head_dim, int gmax, int nw) {
   if (a.bs_shift != 0) return dispatch_block32(a, dtype, head_dim, gmax, nw);
+  if (dtype == VFL_FLOAT32 && a.kvw.slots)  // rows are their own groups here
+    return head_dim == 64 ? valu_fused<64>(a, nw) : valu_fused<128>(a, nw);
   if (dtype == VFL_FLOAT32) {
     if (head_dim == 64) return valu_group<64>(a, gmax, nw);
     if (head_dim == 128) return valu_group<128>(a, gmax, nw);
@@ -370,11 +383,12 @@ static int attention_impl(const void *query, int64_t query_stride_token,
   // Shared-table groups (cross-attention beams) with slot descriptors in group_plan.
   a.desc = nullptr;
   a.desc_stride = 0;
-  if (meta->group_plan != nullptr && !a.own_tables && group_start != nullptr && full_set &&
-      kvw.slots == nullptr) {
-    if ((uintptr_t)meta->group_plan % 16 != 0 ||
+  if (meta->group_plan != nullptr && !a.own_tables && group_start != nullptr &&
+      head_dim_native(head_dim) && block_size == 16 && kvw.slots == nullptr) {
+    const bool bad = (uintptr_t)meta->group_plan % 16 != 0 ||
         meta->group_plan_stride < slot_descriptor_stride(meta->max_blocks_per_seq) ||
-        meta->group_plan_stride % 4 != 0 || meta->group_plan_slots < num_groups) {
+        meta->group_plan_stride % 4 != 0 || meta->group_plan_slots < num_groups;
+    if (bad && full_set) {
       set_error("%s: slot descriptors of %lld slots x %lld words (16-byte aligned, stride at "
                 "least %lld, at least num_groups %lld slots)",
                 who, (long long)meta->group_plan_slots, (long long)meta->group_plan_stride,
@@ -382,8 +396,10 @@ static int attention_impl(const void *query, int64_t query_stride_token,
                 (long long)num_groups);
       return VFL_E_INVALID;
     }
-    a.desc = meta->group_plan;
-    a.desc_stride = meta->group_plan_stride;
+    if (!bad) {  // fp32 launches take them where they fit, and read the call's arrays else
+      a.desc = meta->group_plan;
+      a.desc_stride = meta->group_plan_stride;
+    }
   }
   if (a.own_tables && !full_set) {
     // The VALU kernel and the one-row matrix-core kernel read one table per group; with
@@ -432,9 +448,9 @@ extern "C" int vfl_self_attention_with_kv_write(
               "VFL_GROUP_OWN_TABLES (every row keeps its own block table)");
     return VFL_E_INVALID;
   }
-  if (dtype == VFL_FLOAT32 || !head_dim_native(head_dim) || block_size != 16) {
-    // No fused kernel for fp32, for head sizes other than 64 and 128, or for 32-token
-    // blocks: the same two steps as the reference.
+  if (!head_dim_native(head_dim) || block_size != 16) {
+    // No fused kernel for head sizes other than 64 and 128, or for 32-token blocks: the
+    // same two steps as the reference.
     int st = vfl_reshape_and_cache(key, value, key_stride_token, key_stride_head,
                                    value_stride_token, value_stride_head, k_cache, v_cache,
                                    slot_mapping, num_rows, num_heads, head_dim, block_size,
