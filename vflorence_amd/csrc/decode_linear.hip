@@ -109,41 +109,62 @@ struct LinNorm {
   float2 *y_stats;        // LIN_RESIDUAL: [rows][N / 32] of the stored v
 };
 
-// The workgroup's 32 rows' means and 1/stds from their T tiles' (mean, M2) at
-// st[row * T + t]: thread (row r = tid / 16, j = tid % 16) takes tiles j, j + 16, ...;
-// the 16 threads of a row (one DPP row of a wave) combine them in a fixed order.
+// The workgroup's rows' means and 1/stds from their T tiles' (mean, M2) at
+// st[row * T + t]: thread (row r = tid / TPR, j = tid % TPR) takes tiles j, j + 16, ... and,
+// where 8 threads share a row, j + 8, j + 24, ...; the threads of a row (within one DPP row
+// of a wave) combine them in an order that does not depend on TPR.
 // Requested after the main loop, so the loads' latency overlaps the partial-tile
 // reduction; results in s_ms[r] = (mean, rstd) before the reduction's last barrier.
-struct RowStatLoads {
-  float2 p[2];
+template <int TPR> struct RowStatLoads {
+  static_assert(TPR == 16 || TPR == 8, "16 partial sums per row");
+  static constexpr int H = 16 / TPR;
+  float2 p[H][2];
   __device__ __forceinline__ void issue(const float2 *st, int T, int m0, int M) {
-    const int r = (int)(threadIdx.x >> 4), j = (int)(threadIdx.x & 15);
+    const int r = (int)threadIdx.x / TPR, j0 = (int)threadIdx.x % TPR;
     const float2 *row = st + (int64_t)min(m0 + r, M - 1) * T;
-    p[0] = j < T ? row[j] : make_float2(0.f, 0.f);
-    p[1] = j + 16 < T ? row[j + 16] : make_float2(0.f, 0.f);
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int t = j0 + TPR * h + 16 * i;
+        p[h][i] = t < T ? row[t] : make_float2(0.f, 0.f);
+      }
+  }
+  __device__ __forceinline__ static float total(const float (&s)[H]) {
+    float x = group_sum<TPR>(s[0]);
+    if constexpr (H == 2) x += group_sum<TPR>(s[1]);
+    return x;
   }
   __device__ __forceinline__ void finish(const float2 *st, int T, int m0, int M, float eps,
                                          float2 *s_ms) {
-    const int r = (int)(threadIdx.x >> 4), j = (int)(threadIdx.x & 15);
+    const int r = (int)threadIdx.x / TPR, j0 = (int)threadIdx.x % TPR;
     const float2 *row = st + (int64_t)min(m0 + r, M - 1) * T;
-    float s = p[0].x + p[1].x;
-    for (int t = j + 32; t < T; t += 16) s += row[t].x;
-    const float mean = group_sum<16>(s) / (float)T;
-    float m2 = 0.f;
+    float s[H], m2[H];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      if (j + 16 * i < T) {
-        const float d = p[i].x - mean;
-        m2 += p[i].y + (float)LIN_STAT_TILE * d * d;
+    for (int h = 0; h < H; ++h) {
+      s[h] = p[h][0].x + p[h][1].x;
+      for (int t = j0 + TPR * h + 32; t < T; t += 16) s[h] += row[t].x;
+    }
+    const float mean = total(s) / (float)T;
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      const int j = j0 + TPR * h;
+      m2[h] = 0.f;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        if (j + 16 * i < T) {
+          const float d = p[h][i].x - mean;
+          m2[h] += p[h][i].y + (float)LIN_STAT_TILE * d * d;
+        }
+      }
+      for (int t = j + 32; t < T; t += 16) {
+        const float2 v = row[t];
+        const float d = v.x - mean;
+        m2[h] += v.y + (float)LIN_STAT_TILE * d * d;
       }
     }
-    for (int t = j + 32; t < T; t += 16) {
-      const float2 v = row[t];
-      const float d = v.x - mean;
-      m2 += v.y + (float)LIN_STAT_TILE * d * d;
-    }
-    m2 = group_sum<16>(m2);
-    if (j == 0) s_ms[r] = make_float2(mean, rsqrtf(m2 / (float)(LIN_STAT_TILE * T) + eps));
+    const float q = total(m2);
+    if (j0 == 0) s_ms[r] = make_float2(mean, rsqrtf(q / (float)(LIN_STAT_TILE * T) + eps));
   }
 };
 
@@ -151,28 +172,38 @@ template <int DT> __device__ __forceinline__ float round_elem(float v) {
   return Mfma<DT>::widen(Mfma<DT>::narrow(v));
 }
 
-// LIN_RESIDUAL's epilogue inputs and epilogue.  Finishing wave w < 2 takes token
-// quarter w and both feature quarters of the tile, so each lane holds 8 of a row's 32
-// tile features (4 of each quarter: n0 + 16 f + 4 (lane / 16) .. +3) and the tile row's
-// statistics need only the 4 lanes of the row (rows_sum4), no LDS exchange.
+// The sum of the waves' partial tiles of quarter q, in the order of a 3-level tree: waves
+// w and w + 4 first (SUM4: already added, four sums left), then (s0 + s2) + (s1 + s3).
+template <int SUB, bool SUM4>
+__device__ __forceinline__ floatx4_t sum_partials(const floatx4_t *s_part, int q, int lane) {
+  auto s = [&](int w) {
+    const floatx4_t v = s_part[(w * SUB + q) * 64 + lane];
+    if constexpr (SUM4) return v;
+    else return v + s_part[((w + 4) * SUB + q) * 64 + lane];
+  };
+  return (s(0) + s(2)) + (s(1) + s(3));
+}
+
+// LIN_RESIDUAL's epilogue inputs and epilogue.  Finishing wave w < TT * FT / 2 takes token
+// quarter w % TT and a pair of feature quarters (32 features from n0), so each lane holds 8
+// of a row's 32 statistics-tile features (4 of each quarter: n0 + 16 f + 4 (lane / 16) ..
+// +3) and their statistics need only the 4 lanes of the row (rows_sum4), no LDS exchange.
 struct ResidualIn {
   float b[2][4], r[2][4], g[2][4], be[2][4];  // bias, residual (or its pre-norm sum), LN's
   uint2 raw[2];                               // the residual's 8 values as loaded
   // The residual itself, requested with the operands (its 4 registers are the only ones
   // held through the products).
-  __device__ __forceinline__ void issue_residual(const LinNorm &nrm, int wv, int lane, int m0,
-                                                 int n0, int M) {
-    if (wv >= 2) return;
-    const int64_t row = min(m0 + 16 * wv + (lane & 15), M - 1);
+  __device__ __forceinline__ void issue_residual(const LinNorm &nrm, int lane, int m, int n0,
+                                                 int M) {
+    const int64_t row = min(m, M - 1);
 #pragma unroll
     for (int f = 0; f < 2; ++f)  // n + 3 < N: N is a multiple of 32
       raw[f] = *reinterpret_cast<const uint2 *>(nrm.res + row * nrm.res_stride + n0 + 16 * f +
                                                 4 * (lane >> 4));
   }
   template <int DT>
-  __device__ __forceinline__ void issue(const uint16_t *bias, const LinNorm &nrm, int wv,
-                                        int lane, int n0) {
-    if (wv >= 2) return;
+  __device__ __forceinline__ void issue(const uint16_t *bias, const LinNorm &nrm, int lane,
+                                        int n0) {
 #pragma unroll
     for (int f = 0; f < 2; ++f) {
       const int n = n0 + 16 * f + 4 * (lane >> 4);
@@ -195,14 +226,13 @@ struct ResidualIn {
 
 // The values are rounded where the separate projection store and LayerNorm kernel round
 // them: y, the normalized residual, v.
-template <int DT>
+template <int DT, int FT, int TT, bool SUM4>
 __device__ __forceinline__ void residual_epilogue(const floatx4_t *s_part, int wv, int lane,
                                                   int m0, int n0, int M, int N,
                                                   const ResidualIn &in, const float2 *s_ms,
                                                   uint16_t *y, int64_t ldy, const LinNorm &nrm) {
-  constexpr int SUB = 4, TT = 2;
-  if (wv >= TT) return;
-  const int r = 16 * wv + (lane & 15);  // the workgroup's row
+  const int t = wv % TT, pair = wv / TT;
+  const int r = 16 * t + (lane & 15);  // the workgroup's row
   const int m = m0 + r;
   float mean = 0.f, rstd = 1.f;
   if (nrm.res_stats) {
@@ -212,9 +242,8 @@ __device__ __forceinline__ void residual_epilogue(const floatx4_t *s_part, int w
   float o[2][4];
 #pragma unroll
   for (int f = 0; f < 2; ++f) {
-    const int q = f * TT + wv;  // quarter (feature quarter f, token quarter wv)
-    const floatx4_t v = (s_part[q * 64 + lane] + s_part[(2 * SUB + q) * 64 + lane]) +
-                        (s_part[(SUB + q) * 64 + lane] + s_part[(3 * SUB + q) * 64 + lane]);
+    const floatx4_t v =
+        sum_partials<FT * TT, SUM4>(s_part, (2 * pair + f) * TT + t, lane);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const float yj = round_elem<DT>(v[j] + in.b[f][j]);
@@ -251,22 +280,29 @@ __device__ __forceinline__ void residual_epilogue(const floatx4_t *s_part, int w
 // packed (rows padded to 32; padding rows are left unwritten); PIPE: batches of
 // LIN_PIPE_BATCH steps, double-buffered (for more than LIN_BATCH steps per wave);
 // MODE: LIN_PLAIN, LIN_NORM_IN (x is a pre-norm sum, nrm.x_stats its statistics) or
-// LIN_RESIDUAL (y = v and nrm.y_stats, as described above).
-template <int DT, bool XP, bool GELU, bool YP, bool PIPE, int MODE>
+// LIN_RESIDUAL (y = v and nrm.y_stats, as described above).  FT x TT: 16-feature x 16-token
+// quarters of the output tile (the rule is at pick_tile).
+template <int DT, bool XP, bool GELU, bool YP, bool PIPE, int MODE, int FT, int TT>
 __global__ __launch_bounds__(64 * LIN_WAVES) void decode_linear_kernel(
     const uint16_t *__restrict__ x, int64_t ldx, const uint16_t *__restrict__ wp,
     const uint16_t *__restrict__ bias, uint16_t *__restrict__ y, int64_t ldy, int M, int N,
     int K, bool vec_store, LinNorm nrm) {
   static_assert(MODE != LIN_RESIDUAL || (!GELU && !YP), "the residual epilogue stores v");
   static_assert(MODE != LIN_NORM_IN || !XP, "a pre-norm x is stored row by row");
-  constexpr int FT = LIN_TILE / 16, TT = LIN_TILE / 16;
+  static_assert(!XP || TT == 2, "packed activations are padded to 32 rows");
   constexpr int SUB = FT * TT;  // 16 x 16 quarters of the tile
   constexpr int B = PIPE ? LIN_PIPE_BATCH : LIN_BATCH;
-  // Partial tiles of four waves, each in the MFMA result order (16 bytes per lane).
-  __shared__ floatx4_t s_part[(LIN_WAVES / 2) * SUB * 64];
+  // The 32 x 32 tile, of which a CU holds four, hands the partial tiles over in two halves
+  // (16 KB); the larger ones, one or two on a CU, all at once (64 or 128 KB, one barrier),
+  // and every wave finishes QPW quarters.
+  constexpr bool HALVES = SUB < LIN_WAVES;
+  constexpr int QPW = HALVES ? 1 : SUB / LIN_WAVES;
+  static_assert(TT % QPW == 0, "a wave's quarters share their features");
+  // Partial tiles of four (eight) waves, each in the MFMA result order (16 bytes per lane).
+  __shared__ floatx4_t s_part[(HALVES ? LIN_WAVES / 2 : LIN_WAVES) * SUB * 64];
 
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int n0 = blockIdx.x * LIN_TILE, m0 = blockIdx.y * LIN_TILE;
+  const int n0 = blockIdx.x * (16 * FT), m0 = blockIdx.y * (16 * TT);
   const int ks = K / 32;
   const int kq = K / LIN_WAVES;  // this wave's K range: [wv * kq, (wv + 1) * kq)
   const int kb = wv * kq;
@@ -287,29 +323,29 @@ __global__ __launch_bounds__(64 * LIN_WAVES) void decode_linear_kernel(
                        8 * (lane & 3);
   constexpr int XSTEP = XP ? LIN_BLOCK : 32;
 
-  // Wave q < SUB finishes quarter q of the tile: features 16 (q / TT) + 4 (lane / 16) .. +3
-  // of token 16 (q % TT) + lane % 16.  Its bias is requested now, with the operands, so
-  // that no load is left for after the reduction.
-  static_assert(SUB <= LIN_WAVES, "one quarter per finishing wave");
-  const int qf = wv / TT, qt = wv % TT;
+  // Quarter q of the tile is features 16 (q / TT) + 4 (lane / 16) .. +3 of token
+  // 16 (q % TT) + lane % 16; wave w finishes quarters QPW w .. +QPW - 1.  Their bias is
+  // requested now, with the operands, so that no load is left for after the reduction.
+  const bool finisher = QPW * wv < SUB;
+  const int qf = QPW * wv / TT, qt = QPW * wv % TT;
   const int qn = n0 + 16 * qf + 4 * (lane >> 4);
   float bv[4] = {0.f, 0.f, 0.f, 0.f};
-  if (bias && wv < SUB && MODE == LIN_PLAIN) {
+  if (bias && finisher && MODE == LIN_PLAIN) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) bv[j] = qn + j < N ? Mfma<DT>::widen(bias[qn + j]) : 0.f;
   }
   // The epilogue inputs requested before the operands so that they have landed when
   // the products have (loads complete in order): the rows' tile statistics (two per
   // thread) and, for LIN_NORM_IN's finishing lanes (features qn .. qn + 3), u and b'.
-  __shared__ float2 s_ms[MODE == LIN_PLAIN ? 1 : LIN_TILE];
-  RowStatLoads rsl;
+  __shared__ float2 s_ms[MODE == LIN_PLAIN ? 1 : 16 * TT];
+  RowStatLoads<64 * LIN_WAVES / (16 * TT)> rsl;
   const float2 *row_st = nullptr;
   int row_t = 0;
   float fa[4] = {0.f, 0.f, 0.f, 0.f}, fb[4] = {0.f, 0.f, 0.f, 0.f};  // LIN_NORM_IN: u, b'
   if constexpr (MODE == LIN_NORM_IN) {
     row_st = nrm.x_stats;
     row_t = K / LIN_STAT_TILE;
-    if (wv < SUB) {
+    if (finisher) {
       if (qn + 3 < N && nrm.vec4) {  // one 16-byte load each
         const float4 a = *reinterpret_cast<const float4 *>(nrm.u + qn);
         const float4 b = *reinterpret_cast<const float4 *>(nrm.fbias + qn);
@@ -332,7 +368,11 @@ __global__ __launch_bounds__(64 * LIN_WAVES) void decode_linear_kernel(
   // The residual too, for one batch of K steps (a 1024-deep output projection: 6.2
   // against 6.3 us); a longer, double-buffered K loop ran 0.1 us slower with it here.
   ResidualIn rin;
-  if constexpr (MODE == LIN_RESIDUAL && !PIPE) rin.issue_residual(nrm, wv, lane, m0, n0, M);
+  const bool res_finisher = wv < TT * FT / 2;
+  const int res_m = m0 + 16 * (wv % TT) + (lane & 15), res_n = n0 + 32 * (wv / TT);
+  if constexpr (MODE == LIN_RESIDUAL && !PIPE) {
+    if (res_finisher) rin.issue_residual(nrm, lane, res_m, res_n, M);
+  }
 
   floatx4_t acc[FT][TT];
 #pragma unroll
@@ -393,71 +433,84 @@ __global__ __launch_bounds__(64 * LIN_WAVES) void decode_linear_kernel(
   // below (with them before the operands, a 1024-wide output projection ran 0.3 us
   // slower).
   if constexpr (MODE == LIN_RESIDUAL) {
-    if constexpr (PIPE) rin.issue_residual(nrm, wv, lane, m0, n0, M);
-    rin.issue<DT>(bias, nrm, wv, lane, n0);
+    if (res_finisher) {
+      if constexpr (PIPE) rin.issue_residual(nrm, lane, res_m, res_n, M);
+      rin.issue<DT>(bias, nrm, lane, res_n);
+    }
   }
 
-  // Sum the waves' partial tiles: waves 4..7 hand theirs to waves 0..3, which add and
-  // publish the four sums.
-  if (wv >= LIN_WAVES / 2) {
+  // Sum the waves' partial tiles.  Halves: waves 4..7 hand theirs to waves 0..3, which add
+  // and publish the four sums.
+  if constexpr (!HALVES) {
+#pragma unroll
+    for (int f = 0; f < FT; ++f)
+#pragma unroll
+      for (int t = 0; t < TT; ++t) s_part[(wv * SUB + f * TT + t) * 64 + lane] = acc[f][t];
+  } else if (wv >= LIN_WAVES / 2) {
 #pragma unroll
     for (int f = 0; f < FT; ++f)
 #pragma unroll
       for (int t = 0; t < TT; ++t)
         s_part[((wv - LIN_WAVES / 2) * SUB + f * TT + t) * 64 + lane] = acc[f][t];
   }
-  __syncthreads();
-  if (wv < LIN_WAVES / 2) {
+  if constexpr (HALVES) {
+    __syncthreads();
+    if (wv < LIN_WAVES / 2) {
 #pragma unroll
-    for (int f = 0; f < FT; ++f)
+      for (int f = 0; f < FT; ++f)
 #pragma unroll
-      for (int t = 0; t < TT; ++t) acc[f][t] += s_part[(wv * SUB + f * TT + t) * 64 + lane];
-  }
-  __syncthreads();
-  if (wv < LIN_WAVES / 2) {
+        for (int t = 0; t < TT; ++t) acc[f][t] += s_part[(wv * SUB + f * TT + t) * 64 + lane];
+    }
+    __syncthreads();
+    if (wv < LIN_WAVES / 2) {
 #pragma unroll
-    for (int f = 0; f < FT; ++f)
+      for (int f = 0; f < FT; ++f)
 #pragma unroll
-      for (int t = 0; t < TT; ++t) s_part[(wv * SUB + f * TT + t) * 64 + lane] = acc[f][t];
+        for (int t = 0; t < TT; ++t) s_part[(wv * SUB + f * TT + t) * 64 + lane] = acc[f][t];
+    }
   }
   if (MODE != LIN_PLAIN && row_st)
     rsl.finish(row_st, row_t, m0, M, MODE == LIN_NORM_IN ? nrm.eps : nrm.res_eps, s_ms);
   __syncthreads();
 
-  const int m = m0 + 16 * qt + (lane & 15);
   if constexpr (MODE == LIN_RESIDUAL) {
-    residual_epilogue<DT>(s_part, wv, lane, m0, n0, M, N, rin, s_ms, y, ldy, nrm);
+    if (res_finisher)
+      residual_epilogue<DT, FT, TT, HALVES>(s_part, wv, lane, m0, res_n, M, N, rin, s_ms, y, ldy,
+                                            nrm);
     return;
   }
-  if (wv >= SUB) return;
-  if (qn >= N || m >= M) return;
-  const floatx4_t v = (s_part[wv * 64 + lane] + s_part[(2 * SUB + wv) * 64 + lane]) +
-                      (s_part[(SUB + wv) * 64 + lane] + s_part[(3 * SUB + wv) * 64 + lane]);
-  float mean = 0.f, rstd = 1.f;
-  if constexpr (MODE == LIN_NORM_IN) {
-    const float2 ms = s_ms[16 * qt + (lane & 15)];
-    mean = ms.x;
-    rstd = ms.y;
-  }
-  uint32_t h[4];
+  if (!finisher || qn >= N) return;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const float o = MODE == LIN_NORM_IN ? fmaf(fmaf(-mean, fa[j], v[j]), rstd, fb[j])
-                                        : v[j] + bv[j];
-    h[j] = Mfma<DT>::narrow(GELU ? gelu_of_stored<DT>(o) : o);
-  }
-  if constexpr (YP) {  // 4 consecutive columns of one row: 8 bytes of one lane's chunk
-    *reinterpret_cast<uint2 *>(y + packed_offset(m, qn, N)) =
-        make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
-    return;
-  }
-  uint16_t *dst = y + (int64_t)m * ldy + qn;
-  if (vec_store && qn + 3 < N) {
-    *reinterpret_cast<uint2 *>(dst) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
-  } else {
+  for (int i = 0; i < QPW; ++i) {
+    const int m = m0 + 16 * (qt + i) + (lane & 15);
+    if (m >= M) return;
+    const floatx4_t v = sum_partials<SUB, HALVES>(s_part, QPW * wv + i, lane);
+    float mean = 0.f, rstd = 1.f;
+    if constexpr (MODE == LIN_NORM_IN) {
+      const float2 ms = s_ms[16 * (qt + i) + (lane & 15)];
+      mean = ms.x;
+      rstd = ms.y;
+    }
+    uint32_t h[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (qn + j < N) dst[j] = (uint16_t)h[j];
+    for (int j = 0; j < 4; ++j) {
+      const float o = MODE == LIN_NORM_IN ? fmaf(fmaf(-mean, fa[j], v[j]), rstd, fb[j])
+                                          : v[j] + bv[j];
+      h[j] = Mfma<DT>::narrow(GELU ? gelu_of_stored<DT>(o) : o);
+    }
+    if constexpr (YP) {  // 4 consecutive columns of one row: 8 bytes of one lane's chunk
+      *reinterpret_cast<uint2 *>(y + packed_offset(m, qn, N)) =
+          make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+      continue;
+    }
+    uint16_t *dst = y + (int64_t)m * ldy + qn;
+    if (vec_store && qn + 3 < N) {
+      *reinterpret_cast<uint2 *>(dst) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (qn + j < N) dst[j] = (uint16_t)h[j];
+    }
   }
 }
 
@@ -515,37 +568,78 @@ extern "C" int vfl_pack_linear_weight(const void *weight, int64_t weight_stride,
   return launch_status("pack_linear_weight");
 }
 
-template <bool XP, bool GELU, bool YP, bool PIPE, int MODE>
-static void launch_linear_dt(const dim3 &grid, hipStream_t s, int dtype, const void *x,
-                             int64_t x_stride, const void *wp, const void *bias, void *y,
-                             int64_t y_stride, int64_t rows, int out_features, int in_features,
-                             bool vec_store, const LinNorm &nrm) {
+template <bool XP, bool GELU, bool YP, bool PIPE, int MODE, int FT, int TT>
+static void launch_linear_dt(hipStream_t s, int dtype, const void *x, int64_t x_stride,
+                             const void *wp, const void *bias, void *y, int64_t y_stride,
+                             int64_t rows, int out_features, int in_features, bool vec_store,
+                             const LinNorm &nrm) {
+  const dim3 grid((unsigned)(packed_rows(out_features) / (16 * FT)),
+                  (unsigned)((rows + 16 * TT - 1) / (16 * TT)));
   if (dtype == VFL_BFLOAT16)
-    decode_linear_kernel<VFL_BFLOAT16, XP, GELU, YP, PIPE, MODE>
+    decode_linear_kernel<VFL_BFLOAT16, XP, GELU, YP, PIPE, MODE, FT, TT>
         <<<grid, dim3(64 * LIN_WAVES), 0, s>>>(
         (const uint16_t *)x, x_stride, (const uint16_t *)wp, (const uint16_t *)bias,
         (uint16_t *)y, y_stride, (int)rows, out_features, in_features, vec_store, nrm);
   else
-    decode_linear_kernel<VFL_FLOAT16, XP, GELU, YP, PIPE, MODE>
+    decode_linear_kernel<VFL_FLOAT16, XP, GELU, YP, PIPE, MODE, FT, TT>
         <<<grid, dim3(64 * LIN_WAVES), 0, s>>>(
         (const uint16_t *)x, x_stride, (const uint16_t *)wp, (const uint16_t *)bias,
         (uint16_t *)y, y_stride, (int)rows, out_features, in_features, vec_store, nrm);
 }
 
+enum LinTile { TILE_32x32, TILE_64x32, TILE_64x64 };
+
+// The output tile (features x tokens).  A CU takes two workgroups of 32 x 32 tiles or one of
+// the larger ones, and moves operands at about 30 bytes a cycle whatever their source (the
+// same with the weight in its L2), so what counts is how often the operands are read again
+// -- half as often at 64 x 64 -- and whether the last round of workgroups is full.  Sums
+// run in the same order for every tile: the results are the same bits.
+// - 64 x 64 where 32 x 32 tiles need a second round and it does not, or its second round is
+//   nearly full.  Fused q|k|v and feed-forward of 256 rows, 32 x 32 / 64 x 64, us: 1024 to
+//   3072 9.8 / 9.1, to 4096 12.0 / 10.5, 768 to 3072 8.7 / 7.8; 512 rows to 4096 19.6 / 18.2.
+//   Elsewhere it is the slower one (1024 to 4096: 128 rows 8.2 / 10.4, 384 16.2 / 17.0).
+// - 64 x 32 for the residual projections and depths to 768 where 32 x 32 tiles put a
+//   second workgroup on some CUs: 512 rows, 4096 to 1024 15.8 / 13.4, 1024 to 1024 7.3 / 7.1,
+//   3072 to 768 11.2 / 9.8; 128 rows, 768 to 3072 6.1 / 5.7 (1024 to 3072: 7.3 / 7.4).
+static LinTile pick_tile(int64_t rows, int out_features, int in_features, bool packed_x,
+                         int mode) {
+  if (out_features % 64 != 0) return TILE_32x32;
+  const int64_t t32 = out_features / 32 * ((rows + 31) / 32);
+  const int64_t t64 = out_features / 64 * ((rows + 63) / 64);
+  const bool residual = mode == LIN_RESIDUAL;
+  if (!packed_x && !residual && ((t32 > 512 && t64 <= 256) || (t64 > 448 && t64 <= 512)))
+    return TILE_64x64;
+  if (t32 > 256 && t32 <= 512 && (residual || in_features <= 768)) return TILE_64x32;
+  return TILE_32x32;
+}
+
 // More K steps per wave than one batch holds: double-buffered batches.
 template <bool XP, bool GELU, bool YP, int MODE = LIN_PLAIN>
-static void launch_linear(const dim3 &grid, hipStream_t s, int dtype, const void *x,
-                          int64_t x_stride, const void *wp, const void *bias, void *y,
-                          int64_t y_stride, int64_t rows, int out_features, int in_features,
-                          bool vec_store, const LinNorm &nrm = LinNorm{}) {
-  if (in_features / LIN_WAVES / 32 > LIN_BATCH)
-    launch_linear_dt<XP, GELU, YP, true, MODE>(grid, s, dtype, x, x_stride, wp, bias, y,
-                                               y_stride, rows, out_features, in_features,
-                                               vec_store, nrm);
-  else
-    launch_linear_dt<XP, GELU, YP, false, MODE>(grid, s, dtype, x, x_stride, wp, bias, y,
-                                                y_stride, rows, out_features, in_features,
-                                                vec_store, nrm);
+static void launch_linear(hipStream_t s, int dtype, const void *x, int64_t x_stride,
+                          const void *wp, const void *bias, void *y, int64_t y_stride,
+                          int64_t rows, int out_features, int in_features, bool vec_store,
+                          const LinNorm &nrm = LinNorm{}) {
+  const LinTile tile = pick_tile(rows, out_features, in_features, XP, MODE);
+  const bool pipe = in_features / LIN_WAVES / 32 > LIN_BATCH;
+#define VFL_TILE(P, FT, TT)                                                                  \
+  launch_linear_dt<XP, GELU, YP, P, MODE, FT, TT>(s, dtype, x, x_stride, wp, bias, y, y_stride, \
+                                                  rows, out_features, in_features, vec_store, \
+                                                  nrm)
+  if constexpr (!XP && MODE != LIN_RESIDUAL) {
+    if (tile == TILE_64x64) {
+      if (pipe) VFL_TILE(true, 4, 4);
+      else VFL_TILE(false, 4, 4);
+      return;
+    }
+  }
+  if (tile != TILE_32x32) {
+    if (pipe) VFL_TILE(true, 4, 2);
+    else VFL_TILE(false, 4, 2);
+  } else {
+    if (pipe) VFL_TILE(true, 2, 2);
+    else VFL_TILE(false, 2, 2);
+  }
+#undef VFL_TILE
 }
 
 extern "C" int vfl_linear(const void *x, int64_t x_stride, const void *packed_weight,
@@ -587,12 +681,10 @@ extern "C" int vfl_linear(const void *x, int64_t x_stride, const void *packed_we
     return VFL_E_INVALID;
   }
   const bool vec_store = (uintptr_t)y % 8 == 0 && y_stride % 4 == 0;
-  const dim3 grid((unsigned)(packed_rows(out_features) / LIN_TILE),
-                  (unsigned)((rows + LIN_TILE - 1) / LIN_TILE));
   hipStream_t s = (hipStream_t)stream;
   const bool gelu = flags & VFL_LINEAR_GELU;
 #define VFL_LIN(XP, G, YP)                                                                   \
-  launch_linear<XP, G, YP>(grid, s, dtype, x, x_stride, packed_weight, bias, y, y_stride, rows, \
+  launch_linear<XP, G, YP>(s, dtype, x, x_stride, packed_weight, bias, y, y_stride, rows, \
                            out_features, in_features, vec_store)
   if (!xp && !gelu && !yp)
     VFL_LIN(false, false, false);
@@ -711,11 +803,9 @@ extern "C" int vfl_linear_norm(const void *x, int64_t x_stride, const float *x_s
   nrm.eps = eps;
   nrm.vec4 = ((uintptr_t)u | (uintptr_t)folded_bias) % 16 == 0;
   const bool vec_store = (uintptr_t)y % 8 == 0 && y_stride % 4 == 0;
-  const dim3 grid((unsigned)(packed_rows(out_features) / LIN_TILE),
-                  (unsigned)((rows + LIN_TILE - 1) / LIN_TILE));
   hipStream_t s = (hipStream_t)stream;
 #define VFL_LINN(G, YP)                                                                   \
-  launch_linear<false, G, YP, LIN_NORM_IN>(grid, s, dtype, x, x_stride, packed_weight, nullptr, \
+  launch_linear<false, G, YP, LIN_NORM_IN>(s, dtype, x, x_stride, packed_weight, nullptr, \
                                            y, y_stride, rows, out_features, in_features,     \
                                            vec_store, nrm)
   if (!gelu && !yp)
@@ -785,15 +875,13 @@ extern "C" int vfl_linear_residual(const void *x, int64_t x_stride, const void *
   nrm.res_beta = (const uint16_t *)r_beta;
   nrm.res_eps = r_eps;
   nrm.y_stats = reinterpret_cast<float2 *>(y_stats);
-  const dim3 grid((unsigned)(out_features / LIN_TILE),
-                  (unsigned)((rows + LIN_TILE - 1) / LIN_TILE));
   hipStream_t s = (hipStream_t)stream;
   if (xp)
-    launch_linear<true, false, false, LIN_RESIDUAL>(grid, s, dtype, x, 0, packed_weight, bias, y,
+    launch_linear<true, false, false, LIN_RESIDUAL>(s, dtype, x, 0, packed_weight, bias, y,
                                                     y_stride, rows, out_features, in_features,
                                                     true, nrm);
   else
-    launch_linear<false, false, false, LIN_RESIDUAL>(grid, s, dtype, x, x_stride, packed_weight,
+    launch_linear<false, false, false, LIN_RESIDUAL>(s, dtype, x, x_stride, packed_weight,
                                                      bias, y, y_stride, rows, out_features,
                                                      in_features, true, nrm);
   return launch_status("linear_residual");
