@@ -8,13 +8,13 @@
 // output and the cross-attention query projections).  Each step streams every weight
 // from HBM once (a decoder's weights exceed the last-level cache), so the time goes to
 // memory round trips, not arithmetic: a GEMM that walks K in a loop pays one round
-// trip per K step.  Here a workgroup owns a 32-feature x 32-token output tile and
-// splits K over its 8 waves.  Each wave loads the operands of up to 4 K steps of 32 in
-// one batch, so K <= 1024 costs one round trip; a longer K range is walked in batches
-// of 2 steps with the next batch in flight while one is multiplied.  The waves' partial
-// tiles are summed through LDS in the order of a 3-level tree (waves w and w + 4 first,
-// then (s0 + s2) + (s1 + s3)) with three barriers, and four waves then add the bias and
-// store one 16 x 16 quarter each.
+// trip per K step.  Here a workgroup owns an output tile (32 features x 32 tokens; others
+// by size, see pick_tile) and splits K over its 8 waves.  Each wave loads the operands of
+// up to 4 K steps of 32 in one batch, so K <= 1024 costs one round trip; a longer K range is
+// walked in batches of 2 steps with the next batch in flight while one is multiplied.  The
+// waves' partial tiles are summed through LDS in the order of a 3-level tree (waves w and
+// w + 4 first, then (s0 + s2) + (s1 + s3)), and the waves then add the bias and store a
+// 16 x 16 quarter each.
 //
 // Operand order.  The product per 32-wide K step is mfma_f32_16x16x32 with A = 16
 // weight rows (features) and B = 16 token rows, giving D[feature][token]; a lane's four
@@ -277,21 +277,20 @@ __device__ __forceinline__ void residual_epilogue(const floatx4_t *s_part, int w
 }
 
 // XP: x is packed (no ds_bpermute); GELU: exact GELU after the bias; YP: y is written
-// packed (rows padded to 32; padding rows are left unwritten); PIPE: batches of
-// LIN_PIPE_BATCH steps, double-buffered (for more than LIN_BATCH steps per wave);
+// packed (rows padded to 32; padding rows are left unwritten); B: K steps whose operands
+// are loaded together; PIPE: two such batches, double-buffered;
 // MODE: LIN_PLAIN, LIN_NORM_IN (x is a pre-norm sum, nrm.x_stats its statistics) or
 // LIN_RESIDUAL (y = v and nrm.y_stats, as described above).  FT x TT: 16-feature x 16-token
 // quarters of the output tile (the rule is at pick_tile).
-template <int DT, bool XP, bool GELU, bool YP, bool PIPE, int MODE, int FT, int TT>
+template <int DT, bool XP, bool GELU, bool YP, bool PIPE, int MODE, int FT, int TT, int B>
 __global__ __launch_bounds__(64 * LIN_WAVES) void decode_linear_kernel(
     const uint16_t *__restrict__ x, int64_t ldx, const uint16_t *__restrict__ wp,
     const uint16_t *__restrict__ bias, uint16_t *__restrict__ y, int64_t ldy, int M, int N,
     int K, bool vec_store, LinNorm nrm) {
   static_assert(MODE != LIN_RESIDUAL || (!GELU && !YP), "the residual epilogue stores v");
   static_assert(MODE != LIN_NORM_IN || !XP, "a pre-norm x is stored row by row");
-  static_assert(!XP || TT == 2, "packed activations are padded to 32 rows");
+  static_assert(!XP || TT <= 2, "packed activations are padded to 32 rows");
   constexpr int SUB = FT * TT;  // 16 x 16 quarters of the tile
-  constexpr int B = PIPE ? LIN_PIPE_BATCH : LIN_BATCH;
   // The 32 x 32 tile, of which a CU holds four, hands the partial tiles over in two halves
   // (16 KB); the larger ones, one or two on a CU, all at once (64 or 128 KB, one barrier),
   // and every wave finishes QPW quarters.
@@ -304,8 +303,14 @@ __global__ __launch_bounds__(64 * LIN_WAVES) void decode_linear_kernel(
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int n0 = blockIdx.x * (16 * FT), m0 = blockIdx.y * (16 * TT);
   const int ks = K / 32;
-  const int kq = K / LIN_WAVES;  // this wave's K range: [wv * kq, (wv + 1) * kq)
-  const int kb = wv * kq;
+  // This wave's K steps: wv, wv + 8, ... where it loads them all at once (the waves then
+  // read neighbouring KBs and the two halves of a row's 128-byte lines together: 512 rows,
+  // 1024 to 1024, 6.0 against 7.1 us; 256 rows, 1024 to 4096, 10.0 against 10.5), a
+  // contiguous range of a longer K, walked in batches (4096 to 1024: 10.3 against 10.6).
+  constexpr bool SPREAD = !PIPE && B == LIN_BATCH;
+  constexpr int KSTEP = SPREAD ? LIN_WAVES : 1;
+  const int steps = ks / LIN_WAVES;
+  const int k0 = SPREAD ? wv : wv * steps;
   // byte address of the lane whose 64-byte run holds this lane's operand chunk
   const int src = 4 * (4 * (lane & 15) + (lane >> 4));
 
@@ -315,13 +320,13 @@ __global__ __launch_bounds__(64 * LIN_WAVES) void decode_linear_kernel(
   const uint16_t *xrow[TT];
 #pragma unroll
   for (int f = 0; f < FT; ++f)
-    wblk[f] = wp + ((int64_t)(n0 / 16 + f) * ks + kb / 32) * LIN_BLOCK + lane * 8;
+    wblk[f] = wp + ((int64_t)(n0 / 16 + f) * ks + k0) * LIN_BLOCK + lane * 8;
 #pragma unroll
   for (int t = 0; t < TT; ++t)
-    xrow[t] = XP ? x + ((int64_t)(m0 / 16 + t) * ks + kb / 32) * LIN_BLOCK + lane * 8
-                 : x + (int64_t)min(m0 + 16 * t + (lane >> 2), M - 1) * ldx + kb +
+    xrow[t] = XP ? x + ((int64_t)(m0 / 16 + t) * ks + k0) * LIN_BLOCK + lane * 8
+                 : x + (int64_t)min(m0 + 16 * t + (lane >> 2), M - 1) * ldx + 32 * k0 +
                        8 * (lane & 3);
-  constexpr int XSTEP = XP ? LIN_BLOCK : 32;
+  constexpr int WSTEP = KSTEP * LIN_BLOCK, XSTEP = KSTEP * (XP ? LIN_BLOCK : 32);
 
   // Quarter q of the tile is features 16 (q / TT) + 4 (lane / 16) .. +3 of token
   // 16 (q % TT) + lane % 16; wave w finishes quarters QPW w .. +QPW - 1.  Their bias is
@@ -337,8 +342,9 @@ __global__ __launch_bounds__(64 * LIN_WAVES) void decode_linear_kernel(
   // The epilogue inputs requested before the operands so that they have landed when
   // the products have (loads complete in order): the rows' tile statistics (two per
   // thread) and, for LIN_NORM_IN's finishing lanes (features qn .. qn + 3), u and b'.
-  __shared__ float2 s_ms[MODE == LIN_PLAIN ? 1 : 16 * TT];
-  RowStatLoads<64 * LIN_WAVES / (16 * TT)> rsl;
+  constexpr int TPR = TT > 2 ? 8 : 16;  // threads per row of statistics
+  __shared__ float2 s_ms[MODE == LIN_PLAIN ? 1 : 64 * LIN_WAVES / TPR];
+  RowStatLoads<TPR> rsl;
   const float2 *row_st = nullptr;
   int row_t = 0;
   float fa[4] = {0.f, 0.f, 0.f, 0.f}, fb[4] = {0.f, 0.f, 0.f, 0.f};  // LIN_NORM_IN: u, b'
@@ -380,14 +386,13 @@ __global__ __launch_bounds__(64 * LIN_WAVES) void decode_linear_kernel(
 #pragma unroll
     for (int t = 0; t < TT; ++t) acc[f][t] = floatx4_t{0.f, 0.f, 0.f, 0.f};
 
-  const int steps = kq / 32;
   auto load = [&](uint4 (&a)[B][FT], uint4 (&b)[B][TT], int s0) {
 #pragma unroll
     for (int g = 0; g < B; ++g) {
       if (s0 + g < steps) {
 #pragma unroll
         for (int f = 0; f < FT; ++f)
-          a[g][f] = *reinterpret_cast<const uint4 *>(wblk[f] + LIN_BLOCK * (s0 + g));
+          a[g][f] = *reinterpret_cast<const uint4 *>(wblk[f] + WSTEP * (s0 + g));
 #pragma unroll
         for (int t = 0; t < TT; ++t)
           b[g][t] = *reinterpret_cast<const uint4 *>(xrow[t] + XSTEP * (s0 + g));
@@ -568,7 +573,7 @@ extern "C" int vfl_pack_linear_weight(const void *weight, int64_t weight_stride,
   return launch_status("pack_linear_weight");
 }
 
-template <bool XP, bool GELU, bool YP, bool PIPE, int MODE, int FT, int TT>
+template <bool XP, bool GELU, bool YP, bool PIPE, int MODE, int FT, int TT, int B>
 static void launch_linear_dt(hipStream_t s, int dtype, const void *x, int64_t x_stride,
                              const void *wp, const void *bias, void *y, int64_t y_stride,
                              int64_t rows, int out_features, int in_features, bool vec_store,
@@ -576,68 +581,77 @@ static void launch_linear_dt(hipStream_t s, int dtype, const void *x, int64_t x_
   const dim3 grid((unsigned)(packed_rows(out_features) / (16 * FT)),
                   (unsigned)((rows + 16 * TT - 1) / (16 * TT)));
   if (dtype == VFL_BFLOAT16)
-    decode_linear_kernel<VFL_BFLOAT16, XP, GELU, YP, PIPE, MODE, FT, TT>
+    decode_linear_kernel<VFL_BFLOAT16, XP, GELU, YP, PIPE, MODE, FT, TT, B>
         <<<grid, dim3(64 * LIN_WAVES), 0, s>>>(
         (const uint16_t *)x, x_stride, (const uint16_t *)wp, (const uint16_t *)bias,
         (uint16_t *)y, y_stride, (int)rows, out_features, in_features, vec_store, nrm);
   else
-    decode_linear_kernel<VFL_FLOAT16, XP, GELU, YP, PIPE, MODE, FT, TT>
+    decode_linear_kernel<VFL_FLOAT16, XP, GELU, YP, PIPE, MODE, FT, TT, B>
         <<<grid, dim3(64 * LIN_WAVES), 0, s>>>(
         (const uint16_t *)x, x_stride, (const uint16_t *)wp, (const uint16_t *)bias,
         (uint16_t *)y, y_stride, (int)rows, out_features, in_features, vec_store, nrm);
 }
 
-enum LinTile { TILE_32x32, TILE_64x32, TILE_64x64 };
+enum LinTile { TILE_32x16, TILE_32x32, TILE_64x32, TILE_64x64 };
 
 // The output tile (features x tokens).  A CU takes two workgroups of 32 x 32 tiles or one of
 // the larger ones, and moves operands at about 30 bytes a cycle whatever their source (the
 // same with the weight in its L2), so what counts is how often the operands are read again
 // -- half as often at 64 x 64 -- and whether the last round of workgroups is full.  Sums
 // run in the same order for every tile: the results are the same bits.
+// - 32 x 16 up to 16 rows: half the activation loads.  4 rows against 32 x 32, us: 1024 to
+//   1024 3.7 / 4.2, to 4096 5.7 / 6.0, 4096 to 1024 9.7 / 11.5.
 // - 64 x 64 where 32 x 32 tiles need a second round and it does not, or its second round is
 //   nearly full.  Fused q|k|v and feed-forward of 256 rows, 32 x 32 / 64 x 64, us: 1024 to
-//   3072 9.8 / 9.1, to 4096 12.0 / 10.5, 768 to 3072 8.7 / 7.8; 512 rows to 4096 19.6 / 18.2.
-//   Elsewhere it is the slower one (1024 to 4096: 128 rows 8.2 / 10.4, 384 16.2 / 17.0).
-// - 64 x 32 for the residual projections and depths to 768 where 32 x 32 tiles put a
-//   second workgroup on some CUs: 512 rows, 4096 to 1024 15.8 / 13.4, 1024 to 1024 7.3 / 7.1,
-//   3072 to 768 11.2 / 9.8; 128 rows, 768 to 3072 6.1 / 5.7 (1024 to 3072: 7.3 / 7.4).
-static LinTile pick_tile(int64_t rows, int out_features, int in_features, bool packed_x,
-                         int mode) {
+//   3072 8.7 / 7.5, to 4096 12.2 / 10.0, 768 to 3072 8.7 / 7.8; 512 rows to 4096 19.0 / 17.2.
+//   Elsewhere it is the slower one (1024 to 4096: 128 rows 8.1 / 10.4, 384 15.3 / 16.3).
+// - 64 x 32 where 32 x 32 tiles put a second workgroup on some CUs: 512 rows, 4096 to 1024
+//   15.8 / 13.4, 1024 to 1024 7.4 / 6.1; 128 rows, 768 to 3072 6.1 / 5.5, 1024 to 4096
+//   8.1 / 7.2.  With one on each it loses (256 rows, 1024 to 1024: 5.4 / 5.9).
+static LinTile pick_tile(int64_t rows, int out_features, bool packed_x, int mode) {
+  if (rows <= 16) return TILE_32x16;
   if (out_features % 64 != 0) return TILE_32x32;
   const int64_t t32 = out_features / 32 * ((rows + 31) / 32);
   const int64_t t64 = out_features / 64 * ((rows + 63) / 64);
-  const bool residual = mode == LIN_RESIDUAL;
-  if (!packed_x && !residual && ((t32 > 512 && t64 <= 256) || (t64 > 448 && t64 <= 512)))
+  if (!packed_x && mode != LIN_RESIDUAL &&
+      ((t32 > 512 && t64 <= 256) || (t64 > 448 && t64 <= 512)))
     return TILE_64x64;
-  if (t32 > 256 && t32 <= 512 && (residual || in_features <= 768)) return TILE_64x32;
-  return TILE_32x32;
+  return t32 > 256 && t32 <= 512 ? TILE_64x32 : TILE_32x32;
 }
 
-// More K steps per wave than one batch holds: double-buffered batches.
+// K steps per batch of loads: all of a wave's steps where the registers hold them (4 steps
+// of the larger tiles, 16 of 32 x 16), double-buffered batches beyond.
 template <bool XP, bool GELU, bool YP, int MODE = LIN_PLAIN>
 static void launch_linear(hipStream_t s, int dtype, const void *x, int64_t x_stride,
                           const void *wp, const void *bias, void *y, int64_t y_stride,
                           int64_t rows, int out_features, int in_features, bool vec_store,
                           const LinNorm &nrm = LinNorm{}) {
-  const LinTile tile = pick_tile(rows, out_features, in_features, XP, MODE);
-  const bool pipe = in_features / LIN_WAVES / 32 > LIN_BATCH;
-#define VFL_TILE(P, FT, TT)                                                                  \
-  launch_linear_dt<XP, GELU, YP, P, MODE, FT, TT>(s, dtype, x, x_stride, wp, bias, y, y_stride, \
-                                                  rows, out_features, in_features, vec_store, \
-                                                  nrm)
+  const LinTile tile = pick_tile(rows, out_features, XP, MODE);
+  const int steps = in_features / LIN_K_MULTIPLE;
+#define VFL_TILE(P, FT, TT, B)                                                               \
+  launch_linear_dt<XP, GELU, YP, P, MODE, FT, TT, B>(s, dtype, x, x_stride, wp, bias, y,     \
+                                                     y_stride, rows, out_features,           \
+                                                     in_features, vec_store, nrm)
+  if (tile == TILE_32x16) {
+    if (steps <= LIN_BATCH) VFL_TILE(false, 2, 1, LIN_BATCH);
+    else if (steps <= 16) VFL_TILE(false, 2, 1, 16);
+    else VFL_TILE(true, 2, 1, LIN_BATCH);
+    return;
+  }
   if constexpr (!XP && MODE != LIN_RESIDUAL) {
     if (tile == TILE_64x64) {
-      if (pipe) VFL_TILE(true, 4, 4);
-      else VFL_TILE(false, 4, 4);
+      if (steps > LIN_BATCH) VFL_TILE(true, 4, 4, LIN_PIPE_BATCH);
+      else VFL_TILE(false, 4, 4, LIN_BATCH);
       return;
     }
   }
-  if (tile != TILE_32x32) {
-    if (pipe) VFL_TILE(true, 4, 2);
-    else VFL_TILE(false, 4, 2);
+  if (tile == TILE_64x32) {
+    if (steps > LIN_BATCH) VFL_TILE(true, 4, 2, LIN_PIPE_BATCH);
+    else VFL_TILE(false, 4, 2, LIN_BATCH);
+  } else if (steps <= LIN_BATCH) {
+    VFL_TILE(false, 2, 2, LIN_BATCH);
   } else {
-    if (pipe) VFL_TILE(true, 2, 2);
-    else VFL_TILE(false, 2, 2);
+    VFL_TILE(true, 2, 2, LIN_PIPE_BATCH);
   }
 #undef VFL_TILE
 }
