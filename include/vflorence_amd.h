@@ -436,6 +436,16 @@ int vfl_linear(const void *x, int64_t x_stride, const void *packed_weight, const
                int flags, int dtype, void *stream);
 
 /*
+ * vfl_linear without flags on a weight in its own layout, contiguous
+ * [out_features][in_features] (the encoder's projections, vflorence/models/bart.py:65-75):
+ * out_features a multiple of 32, in_features a multiple of 256 up to 1024, x and weight
+ * 16-byte aligned, the x row stride a multiple of 8 elements.
+ */
+int vfl_linear_rows(const void *x, int64_t x_stride, const void *weight, const void *bias,
+                    void *y, int64_t y_stride, int64_t rows, int out_features, int in_features,
+                    int dtype, void *stream);
+
+/*
  * Deferred LayerNorm across the decoder's projections (no vllm_cpu_attn counterpart:
  * BART's post-LN sublayers, h' = LN(h + y), vflorence/models/bart.py:259-261).
  *

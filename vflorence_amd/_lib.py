@@ -41,6 +41,7 @@ EXPORTED_SYMBOLS = (
     "vfl_linear_packed_elems",
     "vfl_pack_linear_weight",
     "vfl_linear",
+    "vfl_linear_rows",
     "vfl_linear_residual",
     "vfl_linear_norm",
     "vfl_layer_norm_apply",
@@ -127,6 +128,10 @@ _SIGNATURES = {
     "vfl_linear": (
         ctypes.c_int,
         [_vp, _i64, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _i32, _i32, _vp],
+    ),
+    "vfl_linear_rows": (
+        ctypes.c_int,
+        [_vp, _i64, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _i32, _vp],
     ),
     "vfl_linear_residual": (
         ctypes.c_int,

@@ -278,11 +278,13 @@ __device__ __forceinline__ void residual_epilogue(const floatx4_t *s_part, int w
 
 // XP: x is packed (no ds_bpermute); GELU: exact GELU after the bias; YP: y is written
 // packed (rows padded to 32; padding rows are left unwritten); B: K steps whose operands
-// are loaded together; PIPE: two such batches, double-buffered;
+// are loaded together; PIPE: two such batches, double-buffered; WR: the weight is in its own
+// row-major layout, read as the activation rows are;
 // MODE: LIN_PLAIN, LIN_NORM_IN (x is a pre-norm sum, nrm.x_stats its statistics) or
 // LIN_RESIDUAL (y = v and nrm.y_stats, as described above).  FT x TT: 16-feature x 16-token
 // quarters of the output tile (the rule is at pick_tile).
-template <int DT, bool XP, bool GELU, bool YP, bool PIPE, int MODE, int FT, int TT, int B>
+template <int DT, bool XP, bool GELU, bool YP, bool PIPE, int MODE, int FT, int TT, int B,
+          bool WR>
 __global__ __launch_bounds__(64 * LIN_WAVES) void decode_linear_kernel(
     const uint16_t *__restrict__ x, int64_t ldx, const uint16_t *__restrict__ wp,
     const uint16_t *__restrict__ bias, uint16_t *__restrict__ y, int64_t ldy, int M, int N,
@@ -320,13 +322,14 @@ __global__ __launch_bounds__(64 * LIN_WAVES) void decode_linear_kernel(
   const uint16_t *xrow[TT];
 #pragma unroll
   for (int f = 0; f < FT; ++f)
-    wblk[f] = wp + ((int64_t)(n0 / 16 + f) * ks + k0) * LIN_BLOCK + lane * 8;
+    wblk[f] = WR ? wp + (int64_t)(n0 + 16 * f + (lane >> 2)) * K + 32 * k0 + 8 * (lane & 3)
+                 : wp + ((int64_t)(n0 / 16 + f) * ks + k0) * LIN_BLOCK + lane * 8;
 #pragma unroll
   for (int t = 0; t < TT; ++t)
     xrow[t] = XP ? x + ((int64_t)(m0 / 16 + t) * ks + k0) * LIN_BLOCK + lane * 8
                  : x + (int64_t)min(m0 + 16 * t + (lane >> 2), M - 1) * ldx + 32 * k0 +
                        8 * (lane & 3);
-  constexpr int WSTEP = KSTEP * LIN_BLOCK, XSTEP = KSTEP * (XP ? LIN_BLOCK : 32);
+  constexpr int WSTEP = KSTEP * (WR ? 32 : LIN_BLOCK), XSTEP = KSTEP * (XP ? LIN_BLOCK : 32);
 
   // Quarter q of the tile is features 16 (q / TT) + 4 (lane / 16) .. +3 of token
   // 16 (q % TT) + lane % 16; wave w finishes quarters QPW w .. +QPW - 1.  Their bias is
@@ -399,17 +402,20 @@ __global__ __launch_bounds__(64 * LIN_WAVES) void decode_linear_kernel(
       }
     }
   };
+  auto to_operand = [&](uint4 &v) {  // a 64-byte row run in operand order
+    v.x = __builtin_amdgcn_ds_bpermute(src, (int)v.x);
+    v.y = __builtin_amdgcn_ds_bpermute(src, (int)v.y);
+    v.z = __builtin_amdgcn_ds_bpermute(src, (int)v.z);
+    v.w = __builtin_amdgcn_ds_bpermute(src, (int)v.w);
+  };
   auto multiply = [&](uint4 (&a)[B][FT], uint4 (&b)[B][TT], int s0) {
 #pragma unroll
     for (int g = 0; g < B; ++g) {
       if (s0 + g < steps) {
 #pragma unroll
-        for (int t = 0; t < TT && !XP; ++t) {
-          b[g][t].x = __builtin_amdgcn_ds_bpermute(src, (int)b[g][t].x);
-          b[g][t].y = __builtin_amdgcn_ds_bpermute(src, (int)b[g][t].y);
-          b[g][t].z = __builtin_amdgcn_ds_bpermute(src, (int)b[g][t].z);
-          b[g][t].w = __builtin_amdgcn_ds_bpermute(src, (int)b[g][t].w);
-        }
+        for (int t = 0; t < TT && !XP; ++t) to_operand(b[g][t]);
+#pragma unroll
+        for (int f = 0; f < FT && WR; ++f) to_operand(a[g][f]);
 #pragma unroll
         for (int f = 0; f < FT; ++f)
 #pragma unroll
@@ -573,7 +579,8 @@ extern "C" int vfl_pack_linear_weight(const void *weight, int64_t weight_stride,
   return launch_status("pack_linear_weight");
 }
 
-template <bool XP, bool GELU, bool YP, bool PIPE, int MODE, int FT, int TT, int B>
+template <bool XP, bool GELU, bool YP, bool PIPE, int MODE, int FT, int TT, int B,
+          bool WR = false>
 static void launch_linear_dt(hipStream_t s, int dtype, const void *x, int64_t x_stride,
                              const void *wp, const void *bias, void *y, int64_t y_stride,
                              int64_t rows, int out_features, int in_features, bool vec_store,
@@ -581,12 +588,12 @@ static void launch_linear_dt(hipStream_t s, int dtype, const void *x, int64_t x_
   const dim3 grid((unsigned)(packed_rows(out_features) / (16 * FT)),
                   (unsigned)((rows + 16 * TT - 1) / (16 * TT)));
   if (dtype == VFL_BFLOAT16)
-    decode_linear_kernel<VFL_BFLOAT16, XP, GELU, YP, PIPE, MODE, FT, TT, B>
+    decode_linear_kernel<VFL_BFLOAT16, XP, GELU, YP, PIPE, MODE, FT, TT, B, WR>
         <<<grid, dim3(64 * LIN_WAVES), 0, s>>>(
         (const uint16_t *)x, x_stride, (const uint16_t *)wp, (const uint16_t *)bias,
         (uint16_t *)y, y_stride, (int)rows, out_features, in_features, vec_store, nrm);
   else
-    decode_linear_kernel<VFL_FLOAT16, XP, GELU, YP, PIPE, MODE, FT, TT, B>
+    decode_linear_kernel<VFL_FLOAT16, XP, GELU, YP, PIPE, MODE, FT, TT, B, WR>
         <<<grid, dim3(64 * LIN_WAVES), 0, s>>>(
         (const uint16_t *)x, x_stride, (const uint16_t *)wp, (const uint16_t *)bias,
         (uint16_t *)y, y_stride, (int)rows, out_features, in_features, vec_store, nrm);
@@ -718,6 +725,50 @@ extern "C" int vfl_linear(const void *x, int64_t x_stride, const void *packed_we
     VFL_LIN(true, true, true);
 #undef VFL_LIN
   return launch_status("linear");
+}
+
+extern "C" int vfl_linear_rows(const void *x, int64_t x_stride, const void *weight,
+                               const void *bias, void *y, int64_t y_stride, int64_t rows,
+                               int out_features, int in_features, int dtype, void *stream) {
+  clear_error();
+  int st = check_features(out_features, in_features, dtype, "linear_rows");
+  if (st != VFL_OK) return st;
+  if (rows < 0 || x_stride < in_features || y_stride < out_features) {
+    set_error("linear_rows: bad sizes (rows %lld, row strides x %lld y %lld)", (long long)rows,
+              (long long)x_stride, (long long)y_stride);
+    return VFL_E_INVALID;
+  }
+  if (out_features % LIN_TILE != 0 || in_features > LIN_BATCH * LIN_K_MULTIPLE ||
+      rows > 65535LL * 16) {
+    set_error("linear_rows: out_features must be a multiple of %d, in_features and rows at most "
+              "%d and %lld (got %d, %d, %lld)", LIN_TILE, LIN_BATCH * LIN_K_MULTIPLE,
+              65535LL * 16, out_features, in_features, (long long)rows);
+    return VFL_E_UNSUPPORTED;
+  }
+  if (rows == 0) return VFL_OK;
+  if (!x || !weight || !y) {
+    set_error("linear_rows: null pointer argument");
+    return VFL_E_INVALID;
+  }
+  if (((uintptr_t)x | (uintptr_t)weight) % 16 != 0 || x_stride % 8 != 0 ||
+      ((uintptr_t)y | (uintptr_t)bias) % 2 != 0) {
+    set_error("linear_rows: x and the weight must be 16-byte aligned, the x row stride a "
+              "multiple of 8 elements");
+    return VFL_E_INVALID;
+  }
+  const bool vec_store = (uintptr_t)y % 8 == 0 && y_stride % 4 == 0;
+#define VFL_TILE(FT, TT)                                                                     \
+  launch_linear_dt<false, false, false, false, LIN_PLAIN, FT, TT, LIN_BATCH, true>(          \
+      (hipStream_t)stream, dtype, x, x_stride, weight, bias, y, y_stride, rows, out_features, \
+      in_features, vec_store, LinNorm{})
+  switch (pick_tile(rows, out_features, false, LIN_PLAIN)) {
+    case TILE_32x16: VFL_TILE(2, 1); break;
+    case TILE_32x32: VFL_TILE(2, 2); break;
+    case TILE_64x32: VFL_TILE(4, 2); break;
+    case TILE_64x64: VFL_TILE(4, 4); break;
+  }
+#undef VFL_TILE
+  return launch_status("linear_rows");
 }
 
 namespace vfl {

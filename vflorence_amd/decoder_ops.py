@@ -17,7 +17,7 @@ from __future__ import annotations
 import torch
 
 from ._lib import check, lib
-from .hip_attn import _dtype_code, _require_gpu, _stream
+from .hip_attn import _dtype_code, _require_gpu, _stream, plain_eager
 
 # largest k of logprob_topk (each lane keeps its k best in registers)
 MAX_K = 16
@@ -205,6 +205,57 @@ def _(x, packed_weight, bias, out_features, rows=-1, flags=0):
         return x.new_empty(packed_elems(n, out_features))
     lead = (rows,) if flags & LINEAR_X_PACKED else x.shape[:-1]
     return x.new_empty(*lead, out_features)
+
+
+# Where linear_rows takes an eager call, as rows and outputs (rows * out_features).  On the
+# device it is the faster one up to 1024 rows of a 768- or 1024-wide output (590 rows 6.4
+# against 7.6 us for hipBLASLt through torch, 1024 rows 9.2 against 9.4) and 250-400 rows of
+# a q|k|v (256 x 3072 9.2 against 9.3); above that the library call's 19 us of host time, to
+# 7 here, decide until the kernel takes as long (590 x 2304 13.2 us, 455 x 3072 15).
+LINEAR_ROWS_MAX = 1024
+LINEAR_ROWS_MAX_OUTPUTS = 1400000
+
+
+def linear_rows_fits(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> bool:
+    """Whether ``linear_rows`` serves this call of nn.Linear: a plain eager call of 16-bit
+    GPU tensors with rows aligned for its loads, nothing to differentiate."""
+    if (not plain_eager() or torch._C._len_torch_function_stack()
+            or torch.is_autocast_enabled(x.device.type)):
+        return False
+    out_features, in_features = weight.shape
+    if not (type(x) is torch.Tensor and x.is_cuda and x.dim() == 2
+            and x.dtype in (torch.bfloat16, torch.float16)
+            and weight.dtype == x.dtype and weight.device == x.device
+            and type(weight) in (torch.Tensor, torch.nn.Parameter)
+            and x.shape[1] == in_features
+            and 0 < x.shape[0] <= LINEAR_ROWS_MAX
+            and x.shape[0] * out_features <= LINEAR_ROWS_MAX_OUTPUTS
+            and out_features % 64 == 0 and in_features % LINEAR_K_MULTIPLE == 0
+            and in_features <= 1024):
+        return False
+    if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad
+                                    or (bias is not None and bias.requires_grad)):
+        return False
+    if bias is not None and not (bias.dtype == x.dtype and bias.device == x.device
+                                 and type(bias) in (torch.Tensor, torch.nn.Parameter)
+                                 and bias.shape == (out_features,) and bias.is_contiguous()):
+        return False
+    return (x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= in_features
+            and x.data_ptr() % 16 == 0 and weight.is_contiguous()
+            and weight.data_ptr() % 16 == 0)
+
+
+def linear_rows(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
+    """``x @ weight.T + bias`` for calls that ``linear_rows_fits`` accepts, from the weight's
+    own layout (``vfl_linear_rows``)."""
+    rows, in_features = x.shape
+    out_features = weight.shape[0]
+    out = x.new_empty(rows, out_features)
+    check(lib.vfl_linear_rows(x.data_ptr(), x.stride(0), weight.data_ptr(),
+                              None if bias is None else bias.data_ptr(), out.data_ptr(),
+                              out_features, rows, out_features, in_features,
+                              _dtype_code(x.dtype), _stream(x.device)))
+    return out
 
 
 # Deferred LayerNorm (vfl_linear_residual / vfl_linear_norm / vfl_layer_norm_apply): a

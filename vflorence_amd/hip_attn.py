@@ -682,6 +682,15 @@ def self_attention_with_kv_write(
     )
 
 
+def plain_eager() -> bool:
+    """Whether nothing traces, batches, differentiates forward or intercepts operators, so
+    that a kernel call outside the dispatcher does what its operator would."""
+    return not (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
+                or torch._C._len_torch_dispatch_stack()
+                or torch._C._functorch.maybe_current_level() is not None
+                or torch.autograd.forward_ad._current_level >= 0)
+
+
 ENCODER_HEAD_DIM = 64  # head size of the packed encoder attention kernel
 
 
@@ -695,11 +704,7 @@ def encoder_attention_fits(qkv: torch.Tensor, out: torch.Tensor | None, num_head
             and qkv.dim() == 2 and qkv.shape[1] == 3 * num_heads * ENCODER_HEAD_DIM
             and scale > 0):
         return False
-    if (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
-            or torch._C._len_torch_dispatch_stack()
-            or torch._C._functorch.maybe_current_level() is not None
-            or torch.autograd.forward_ad._current_level >= 0
-            or (qkv.requires_grad and torch.is_grad_enabled())):
+    if not plain_eager() or (qkv.requires_grad and torch.is_grad_enabled()):
         return False
     if qkv.stride(1) != 1 or qkv.stride(0) % 8 or qkv.data_ptr() % 16:
         return False

@@ -267,13 +267,26 @@ def _runs_fit(segments, rows: int) -> bool:
     return at <= rows
 
 
+class EncoderLinear(nn.Linear):
+    """nn.Linear whose small eager 16-bit calls run the split-K kernel on the weight as it
+    is (``decoder_ops.linear_rows``): there the library call is all host time."""
+
+    def forward(self, x: torch.Tensor) -> torch.Tensor:
+        if x.is_cuda:
+            from .. import decoder_ops
+
+            if decoder_ops.linear_rows_fits(x, self.weight, self.bias):
+                return decoder_ops.linear_rows(x, self.weight, self.bias)
+        return super().forward(x)
+
+
 class BartEncoderSelfAttention(_Heads):
     fused_projections = {"qkv_proj": ("q_proj", "k_proj", "v_proj")}
 
     def __init__(self, embed_dim: int, num_heads: int):
         super().__init__(embed_dim, num_heads)
-        self.qkv_proj = nn.Linear(embed_dim, 3 * embed_dim)
-        self.out_proj = nn.Linear(embed_dim, embed_dim)
+        self.qkv_proj = EncoderLinear(embed_dim, 3 * embed_dim)
+        self.out_proj = EncoderLinear(embed_dim, embed_dim)
 
     def attention(self, x: torch.Tensor, segments=None) -> torch.Tensor:
         """Attention output before ``out_proj``.  ``x``: [B, S, d] equal-length prompts,
