@@ -186,10 +186,11 @@ int vfl_build_group_plan(const int32_t *block_table, int64_t block_table_stride,
  * group_order is NULL) as [first row, rows, seq_lens[first row], 0, block_table[first
  * row][0 .. max_blocks_per_seq)], later slots [0, 0, 0, 0].  Passed (device copy) as
  * vfl_sched_meta.group_plan with VFL_GROUP_SHARED_TABLE groups and group_plan_stride /
- * group_plan_slots set, vfl_attention_with_kv_cache's 16-bit head-size-64/128 launch
- * reads each workgroup's group from its slot in one dependent load instead of three
- * (dispatch order, group start, then length and table); the call's group_start,
- * group_order, seq_lens and block_table must describe the same groups.
+ * group_plan_slots set, vfl_attention_with_kv_cache's head-size-64/128 launch over
+ * 16-token blocks reads each workgroup's group from its slot in one dependent load instead
+ * of three (dispatch order, group start, then length and table); the call's group_start,
+ * group_order, seq_lens and block_table must describe the same groups.  fp32 launches
+ * ignore descriptors of too few slots or too short a stride, 16-bit ones refuse them.
  */
 int64_t vfl_slot_descriptor_stride(int64_t max_blocks_per_seq);
 int vfl_build_slot_descriptors(const int32_t *block_table, int64_t block_table_stride,
@@ -425,7 +426,7 @@ enum vfl_linear_flags {
  * in_features a multiple of 256 (and out_features of 32 for a packed output); rows at
  * most 65535 * 32.  x and `packed` 16-byte aligned; an unpacked x has a row stride
  * (elements) that is a multiple of 8 and at least in_features.  Split-K over the 8
- * waves of a workgroup per 32 x 32 output tile: one memory round trip for the weight
+ * waves of a workgroup per output tile (32 x 16 to 64 x 64): one memory round trip for the weight
  * when in_features <= 1024.
  */
 int64_t vfl_linear_packed_elems(int rows, int cols);

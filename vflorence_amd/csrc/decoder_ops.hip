@@ -6,7 +6,7 @@
 //   logprob_topk_kernel    -- per row: log-softmax of the logits, the generation rules
 //                             (min length, forced BOS / EOS, suppressed tokens), and the
 //                             k best (score, token) pairs, best first; one read of the
-//                             logits.  With log_softmax off the scores are the processed
+//                             logits (logprob_topk_row_kernel), two for very long rows.  With log_softmax off the scores are the processed
 //                             logits themselves (greedy decoding's argmax at k = 1).
 //
 // Both are bandwidth-bound streams over [rows, dim] / [rows, vocab] in HBM.
