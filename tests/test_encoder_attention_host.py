@@ -7,7 +7,7 @@ import torch
 
 from vflorence_amd import hip_attn
 from vflorence_amd._lib import lib
-from vflorence_amd.layers.bart import _runs_fit
+from vflorence_amd.layers.bart import BartEncoderSelfAttention, _runs_fit
 
 
 def call(segments=((0, 1, 4),), heads=2, dim=64, stride=384, scale=0.125, dtype=1, tokens=4,
@@ -33,3 +33,18 @@ def test_runs_and_plain_calls():
     assert not _runs_fit([(0, 2, 3)], 5) and not _runs_fit([(3, 1, 2), (0, 1, 2)], 9)
     assert not hip_attn.encoder_attention_fits(torch.zeros(4, 384, dtype=torch.bfloat16), None, 2,
                                                0.125)
+
+
+def test_runs_given_once(monkeypatch):
+    """Runs from a one-shot iterable reach the kernel as the same runs in a list do."""
+    seen = []
+    monkeypatch.setattr(hip_attn, "encoder_attention_fits", lambda *a: True)
+    monkeypatch.setattr(hip_attn, "encoder_attention",
+                        lambda qkv, segments, *a: seen.append([tuple(r) for r in segments]))
+    runs = [(0, 2, 3), (6, 1, 4)]
+    layer, qkv, out = BartEncoderSelfAttention(128, 2), torch.zeros(10, 384), torch.zeros(10, 128)
+    layer.attend(qkv, runs, out)
+    layer.attend(qkv, iter(runs), out)
+    layer.attend(qkv, zip(*zip(*runs)), out)
+    layer.attend(qkv, (map(int, r) for r in runs), out)
+    assert seen == [runs] * 4

@@ -315,6 +315,7 @@ class BartEncoderSelfAttention(_Heads):
         ``qkv`` [>= T, 3 d], written to rows ``start .. start + count * length`` of
         ``out``; other rows are left as they are.  One launch for all runs where the
         packed kernel serves the call (hip_attn.encoder_attention_fits), else SDPA per run."""
+        segments = [tuple(run) for run in segments]  # read more than once below
         if (hip_attn.encoder_attention_fits(qkv, out, self.num_heads, self.scaling)
                 and _runs_fit(segments, min(qkv.shape[0], out.shape[0]))):
             hip_attn.encoder_attention(qkv, segments, out, self.num_heads, self.scaling)
