@@ -493,7 +493,8 @@ int vfl_layer_norm_apply(const void *v, int64_t v_stride, const float *v_stats,
  * `start` on, within the num_tokens rows; rows that no segment names are neither read nor
  * written.  q, k and v: rows of num_heads x head_dim elements at one row stride (the
  * thirds of a fused q|k|v projection), 16-byte aligned, the stride a multiple of 8; out
- * 8-byte aligned, its stride a multiple of 4.  bf16 and fp16, head_dim 64 (else
+ * 8-byte aligned, its stride a multiple of 4, overlapping none of q, k and v.  bf16 and
+ * fp16, head_dim 64 (else
  * VFL_E_UNSUPPORTED), scale > 0.  Scores, softmax and sums in fp32, the weights rounded to
  * the element type for the second product.  One launch per 128 segments.
  */

@@ -76,3 +76,20 @@ def test_layer_forms():
     assert layer.qkv_proj.weight.grad is not None
     c = c.detach()
     assert float((a - c).float().norm() / c.float().norm()) < 1e-2  # two bf16 roundings
+
+
+@pytest.mark.parametrize("third", [0, 1, 2])
+def test_output_over_the_projections(third):
+    """An output that overlaps q, k or v keeps torch's path: its rows are complete before
+    any is stored."""
+    g = torch.Generator(device="cuda").manual_seed(third)
+    layer = BartEncoderSelfAttention(128, 2).cuda().to(torch.bfloat16)
+    qkv = torch.randn(700, 384, generator=g, device="cuda").to(torch.bfloat16)
+    want, runs = torch.empty(700, 128, dtype=qkv.dtype, device="cuda"), [(0, 1, 600), (600, 2, 50)]
+    out = qkv[:, 128 * third:128 * (third + 1)]
+    with torch.no_grad():
+        assert hip_attn.encoder_attention_fits(qkv, want, 2, 0.125)
+        assert not hip_attn.encoder_attention_fits(qkv, out, 2, 0.125)
+        before = qkv.clone()
+        layer.attend(qkv, runs, out)
+    check(out.clone(), before, runs, 2)

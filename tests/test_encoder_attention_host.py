@@ -48,3 +48,13 @@ def test_runs_given_once(monkeypatch):
     layer.attend(qkv, zip(*zip(*runs)), out)
     layer.attend(qkv, (map(int, r) for r in runs), out)
     assert seen == [runs] * 4
+
+
+def test_shared_memory_is_seen():
+    rows = torch.zeros(12, 512, dtype=torch.bfloat16)
+    other = torch.zeros(12, 128, dtype=torch.bfloat16)
+    meet = hip_attn._spans_meet
+    assert meet(rows[:, :384], rows[:, 128:256]) and meet(rows[:, 256:384], rows[:, :384])
+    assert meet(rows[:6, :384], rows[4:, 384:]) and meet(rows[:1], rows[:1])
+    assert not meet(rows[:6], rows[6:]) and not meet(rows[6:], rows[:6])
+    assert not meet(rows, other) and not meet(other, rows)

@@ -694,11 +694,21 @@ def plain_eager() -> bool:
 ENCODER_HEAD_DIM = 64  # head size of the packed encoder attention kernel
 
 
+def _spans_meet(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether the address ranges of two non-empty [rows, columns] tensors of unit column
+    stride meet (interleaved columns of one buffer count as meeting)."""
+    a0, b0 = a.data_ptr(), b.data_ptr()
+    a1 = a0 + ((a.shape[0] - 1) * a.stride(0) + a.shape[1]) * a.element_size()
+    b1 = b0 + ((b.shape[0] - 1) * b.stride(0) + b.shape[1]) * b.element_size()
+    return a0 < b1 and b0 < a1
+
+
 def encoder_attention_fits(qkv: torch.Tensor, out: torch.Tensor | None, num_heads: int,
                            scale: float) -> bool:
     """Whether ``encoder_attention`` serves these ``[tokens, 3 d]`` projections: 16-bit GPU
     tensors of 64-wide heads whose rows are aligned for its loads, in a plain eager call
-    (nothing to differentiate, trace, batch or dispatch elsewhere)."""
+    (nothing to differentiate, trace, batch or dispatch elsewhere), with an ``out`` that
+    shares no memory with them: a workgroup stores its rows while others still read."""
     if not (type(qkv) is torch.Tensor and qkv.is_cuda
             and qkv.dtype in (torch.bfloat16, torch.float16)
             and qkv.dim() == 2 and qkv.shape[1] == 3 * num_heads * ENCODER_HEAD_DIM
@@ -713,7 +723,8 @@ def encoder_attention_fits(qkv: torch.Tensor, out: torch.Tensor | None, num_head
                            and not out.requires_grad
                            and out.shape[1] == num_heads * ENCODER_HEAD_DIM
                            and out.stride(1) == 1 and out.stride(0) % 4 == 0
-                           and out.stride(0) >= out.shape[1] and out.data_ptr() % 8 == 0)
+                           and out.stride(0) >= out.shape[1] and out.data_ptr() % 8 == 0
+                           and not _spans_meet(qkv, out))
 
 
 def encoder_attention(qkv: torch.Tensor, segments, out: torch.Tensor, num_heads: int,
