@@ -3,7 +3,7 @@
 import pytest
 import torch
 
-from vflorence_amd import hip_attn
+from vflorence_amd import decoder_ops, hip_attn
 from vflorence_amd.layers.bart import BartEncoderSelfAttention
 
 pytestmark = pytest.mark.gpu
@@ -93,3 +93,16 @@ def test_output_over_the_projections(third):
         before = qkv.clone()
         layer.attend(qkv, runs, out)
     check(out.clone(), before, runs, 2)
+
+
+def test_tensors_of_another_device(monkeypatch):
+    """Neither the attention nor the projections launch their own kernels for tensors of a
+    device that is not current."""
+    layer = BartEncoderSelfAttention(256, 4).cuda().to(torch.bfloat16)
+    x = torch.randn(40, 256, device="cuda").to(torch.bfloat16)
+    calls = lambda: (hip_attn.encoder_attention_fits(layer.qkv_proj(x), None, 4, 0.125),  # noqa: E731
+                     decoder_ops.linear_rows_fits(x, layer.out_proj.weight, layer.out_proj.bias))
+    with torch.no_grad():
+        assert calls() == (True, True)
+        monkeypatch.setattr(torch.cuda, "current_device", lambda: x.get_device() + 1)
+        assert calls() == (False, False)

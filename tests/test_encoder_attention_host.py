@@ -1,6 +1,7 @@
 """vfl_encoder_attention's argument checks and the calls that keep torch's path (CPU)."""
 
 import ctypes
+from types import SimpleNamespace
 
 import pytest
 import torch
@@ -58,3 +59,9 @@ def test_shared_memory_is_seen():
     assert meet(rows[:6, :384], rows[4:, 384:]) and meet(rows[:1], rows[:1])
     assert not meet(rows[:6], rows[6:]) and not meet(rows[6:], rows[:6])
     assert not meet(rows, other) and not meet(other, rows)
+
+
+def test_current_device(monkeypatch):
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    for index in (0, 1):
+        assert hip_attn.on_current_device(SimpleNamespace(get_device=lambda: index)) == index

@@ -17,7 +17,7 @@ from __future__ import annotations
 import torch
 
 from ._lib import check, lib
-from .hip_attn import _dtype_code, _require_gpu, _stream, plain_eager
+from .hip_attn import _dtype_code, _require_gpu, _stream, on_current_device, plain_eager
 
 # largest k of logprob_topk (each lane keeps its k best in registers)
 MAX_K = 16
@@ -218,12 +218,12 @@ LINEAR_ROWS_MAX_OUTPUTS = 1400000
 
 def linear_rows_fits(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> bool:
     """Whether ``linear_rows`` serves this call of nn.Linear: a plain eager call of 16-bit
-    GPU tensors with rows aligned for its loads, nothing to differentiate."""
+    tensors on the current GPU with rows aligned for its loads, nothing to differentiate."""
     if (not plain_eager() or torch._C._len_torch_function_stack()
             or torch.is_autocast_enabled(x.device.type)):
         return False
     out_features, in_features = weight.shape
-    if not (type(x) is torch.Tensor and x.is_cuda and x.dim() == 2
+    if not (type(x) is torch.Tensor and x.is_cuda and on_current_device(x) and x.dim() == 2
             and x.dtype in (torch.bfloat16, torch.float16)
             and weight.dtype == x.dtype and weight.device == x.device
             and type(weight) in (torch.Tensor, torch.nn.Parameter)

@@ -703,18 +703,25 @@ def _spans_meet(a: torch.Tensor, b: torch.Tensor) -> bool:
     return a0 < b1 and b0 < a1
 
 
+def on_current_device(tensor: torch.Tensor) -> bool:
+    """Whether a GPU tensor is on the current device.  A launch outside the dispatcher goes
+    to the current device where the stream handle is null, as every default stream's is."""
+    return tensor.get_device() == torch.cuda.current_device()
+
+
 def encoder_attention_fits(qkv: torch.Tensor, out: torch.Tensor | None, num_heads: int,
                            scale: float) -> bool:
-    """Whether ``encoder_attention`` serves these ``[tokens, 3 d]`` projections: 16-bit GPU
-    tensors of 64-wide heads whose rows are aligned for its loads, in a plain eager call
-    (nothing to differentiate, trace, batch or dispatch elsewhere), with an ``out`` that
+    """Whether ``encoder_attention`` serves these ``[tokens, 3 d]`` projections: 16-bit
+    tensors of 64-wide heads on the current GPU whose rows are aligned for its loads, in a
+    plain eager call (nothing to differentiate, trace, batch or dispatch elsewhere), with an ``out`` that
     shares no memory with them: a workgroup stores its rows while others still read."""
     if not (type(qkv) is torch.Tensor and qkv.is_cuda
             and qkv.dtype in (torch.bfloat16, torch.float16)
             and qkv.dim() == 2 and qkv.shape[1] == 3 * num_heads * ENCODER_HEAD_DIM
             and scale > 0):
         return False
-    if not plain_eager() or (qkv.requires_grad and torch.is_grad_enabled()):
+    if (not plain_eager() or not on_current_device(qkv)
+            or (qkv.requires_grad and torch.is_grad_enabled())):
         return False
     if qkv.stride(1) != 1 or qkv.stride(0) % 8 or qkv.data_ptr() % 16:
         return False
