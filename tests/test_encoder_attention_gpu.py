@@ -106,3 +106,25 @@ def test_tensors_of_another_device(monkeypatch):
         assert calls() == (True, True)
         monkeypatch.setattr(torch.cuda, "current_device", lambda: x.get_device() + 1)
         assert calls() == (False, False)
+
+
+def test_function_modes_see_the_call():
+    from torch.overrides import TorchFunctionMode
+
+    class Names(TorchFunctionMode):
+        def __init__(self):
+            super().__init__()
+            self.names = set()
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            self.names.add(getattr(func, "__name__", ""))
+            return func(*args, **(kwargs or {}))
+
+    layer = BartEncoderSelfAttention(256, 4).cuda().to(torch.bfloat16)
+    x = torch.randn(2, 40, 256, device="cuda").to(torch.bfloat16)
+    with torch.no_grad(), Names() as seen:
+        layer(x)
+        assert {"linear", "scaled_dot_product_attention"} <= seen.names
+        seen.names.clear()
+        layer(x.view(-1, 256), [(0, 2, 40)])
+        assert {"linear", "scaled_dot_product_attention"} <= seen.names

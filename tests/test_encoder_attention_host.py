@@ -65,3 +65,20 @@ def test_current_device(monkeypatch):
     monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
     for index in (0, 1):
         assert hip_attn.on_current_device(SimpleNamespace(get_device=lambda: index)) == index
+
+
+def test_modes_are_not_passed_by():
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    assert hip_attn.plain_eager()
+    with torch.device("cpu"):  # a default device: a function mode that takes no operator
+        assert hip_attn.plain_eager()
+    for mode in (TorchFunctionMode, TorchDispatchMode):
+        with mode():
+            assert not hip_attn.plain_eager()
+    seen = []
+    torch.vmap(lambda x: seen.append(hip_attn.plain_eager()) or x)(torch.zeros(2))
+    with torch.autograd.forward_ad.dual_level():
+        seen.append(hip_attn.plain_eager())
+    assert seen == [False, False] and hip_attn.plain_eager()

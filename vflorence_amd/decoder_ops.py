@@ -219,8 +219,7 @@ LINEAR_ROWS_MAX_OUTPUTS = 1400000
 def linear_rows_fits(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> bool:
     """Whether ``linear_rows`` serves this call of nn.Linear: a plain eager call of 16-bit
     tensors on the current GPU with rows aligned for its loads, nothing to differentiate."""
-    if (not plain_eager() or torch._C._len_torch_function_stack()
-            or torch.is_autocast_enabled(x.device.type)):
+    if not plain_eager() or torch.is_autocast_enabled(x.device.type):
         return False
     out_features, in_features = weight.shape
     if not (type(x) is torch.Tensor and x.is_cuda and on_current_device(x) and x.dim() == 2

@@ -15,6 +15,8 @@ import ctypes
 from dataclasses import dataclass, field
 
 import torch
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import _lib
 from ._lib import SchedMeta, check, lib
@@ -682,11 +684,18 @@ def self_attention_with_kv_write(
     )
 
 
+def _functions_intercepted() -> bool:
+    """Whether a torch function mode other than a default device (which acts on factory
+    calls alone) is active."""
+    return any(type(mode) is not DeviceContext for mode in _get_current_function_mode_stack())
+
+
 def plain_eager() -> bool:
     """Whether nothing traces, batches, differentiates forward or intercepts operators, so
     that a kernel call outside the dispatcher does what its operator would."""
     return not (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
                 or torch._C._len_torch_dispatch_stack()
+                or (torch._C._len_torch_function_stack() and _functions_intercepted())
                 or torch._C._functorch.maybe_current_level() is not None
                 or torch.autograd.forward_ad._current_level >= 0)
 
