@@ -128,3 +128,16 @@ def test_function_modes_see_the_call():
         seen.names.clear()
         layer(x.view(-1, 256), [(0, 2, 40)])
         assert {"linear", "scaled_dot_product_attention"} <= seen.names
+
+
+def test_overlapping_rows():
+    """Projections whose rows overlap (expanded, or a window that slides by less than a
+    row) keep torch's path instead of the kernel's refusal."""
+    layer = BartEncoderSelfAttention(128, 2).cuda().to(torch.bfloat16)
+    flat = torch.randn(384 * 40, device="cuda").to(torch.bfloat16)
+    for qkv in (flat[:384].expand(40, 384), flat.as_strided((40, 384), (8, 1))):
+        out = torch.empty(40, 128, dtype=qkv.dtype, device="cuda")
+        with torch.no_grad():
+            assert not hip_attn.encoder_attention_fits(qkv, out, 2, 0.125)
+            layer.attend(qkv, [(0, 1, 40)], out)
+        check(out, qkv.contiguous(), [(0, 1, 40)], 2)

@@ -732,7 +732,8 @@ def encoder_attention_fits(qkv: torch.Tensor, out: torch.Tensor | None, num_head
     if (not plain_eager() or not on_current_device(qkv)
             or (qkv.requires_grad and torch.is_grad_enabled())):
         return False
-    if qkv.stride(1) != 1 or qkv.stride(0) % 8 or qkv.data_ptr() % 16:
+    if (qkv.stride(1) != 1 or qkv.stride(0) % 8 or qkv.stride(0) < qkv.shape[1]
+            or qkv.data_ptr() % 16):
         return False
     return out is None or (type(out) is torch.Tensor and out.device == qkv.device
                            and out.dtype == qkv.dtype and out.dim() == 2
