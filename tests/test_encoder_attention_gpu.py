@@ -141,3 +141,12 @@ def test_overlapping_rows():
             assert not hip_attn.encoder_attention_fits(qkv, out, 2, 0.125)
             layer.attend(qkv, [(0, 1, 40)], out)
         check(out, qkv.contiguous(), [(0, 1, 40)], 2)
+
+
+def test_empty_run_of_a_long_length():
+    layer = BartEncoderSelfAttention(128, 2).cuda().to(torch.bfloat16)
+    qkv = torch.randn(40, 384, device="cuda").to(torch.bfloat16)
+    out = torch.empty(40, 128, dtype=qkv.dtype, device="cuda")
+    with torch.no_grad():
+        layer.attend(qkv, [(0, 1, 30), (30, 0, 1000), (30, 1, 10)], out)
+    check(out, qkv, [(0, 1, 30), (30, 1, 10)], 2)

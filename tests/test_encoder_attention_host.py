@@ -82,3 +82,16 @@ def test_modes_are_not_passed_by():
     with torch.autograd.forward_ad.dual_level():
         seen.append(hip_attn.plain_eager())
     assert seen == [False, False] and hip_attn.plain_eager()
+
+
+def test_runs_of_no_tokens(monkeypatch):
+    """A run of no prompts may state any length, as torch's path allows."""
+    seen = []
+    fake = SimpleNamespace(vfl_encoder_attention=lambda *a: seen.append(a[7][:3 * a[8]]) or 0)
+    monkeypatch.setattr(hip_attn, "lib", fake)
+    monkeypatch.setattr(hip_attn, "_stream", lambda device: 0)
+    qkv, out = torch.zeros(10, 384).bfloat16(), torch.zeros(10, 128).bfloat16()
+    runs = [(0, 2, 3), (6, 0, 1000), (6, 1, 4), (10, 0, 1 << 70), (10, 5, 0)]
+    assert _runs_fit(runs, 10)
+    hip_attn.encoder_attention(qkv, runs, out, 2, 0.125)
+    assert seen == [[0, 2, 3, 6, 1, 4]]

@@ -748,12 +748,12 @@ def encoder_attention(qkv: torch.Tensor, segments, out: torch.Tensor, num_heads:
                       scale: float) -> None:
     """Self-attention of packed prompts (``vfl_encoder_attention``): ``qkv`` ``[tokens, 3 d]``
     holds each token's q, k and v, ``segments`` lists ``(start, count, length)`` runs of
-    equal-length prompts, and the rows they name of ``out`` ``[tokens, d]`` are written.
-    For calls that ``encoder_attention_fits`` accepts."""
+    equal-length prompts, and the rows they name of ``out`` ``[tokens, d]`` are written;
+    runs of no tokens are left out, whatever length they state.  For calls that ``encoder_attention_fits`` accepts."""
     tokens = min(qkv.shape[0], out.shape[0])
     if tokens == 0:
         return
-    flat = [int(x) for run in segments for x in run]
+    flat = [int(x) for run in segments if run[1] and run[2] for x in run]
     triples = (ctypes.c_int64 * len(flat))(*flat)
     d, base, size = num_heads * ENCODER_HEAD_DIM, qkv.data_ptr(), qkv.element_size()
     check(lib.vfl_encoder_attention(
