@@ -95,3 +95,5 @@ def test_runs_of_no_tokens(monkeypatch):
     assert _runs_fit(runs, 10)
     hip_attn.encoder_attention(qkv, runs, out, 2, 0.125)
     assert seen == [[0, 2, 3, 6, 1, 4]]
+    with pytest.raises(TypeError):  # as a slice by it is
+        hip_attn.encoder_attention(qkv, [(0, 1, 4.5)], out, 2, 0.125)

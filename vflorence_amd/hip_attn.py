@@ -12,6 +12,7 @@ tensors are rejected: there is no host implementation behind these names.
 from __future__ import annotations
 
 import ctypes
+import operator
 from dataclasses import dataclass, field
 
 import torch
@@ -753,7 +754,7 @@ def encoder_attention(qkv: torch.Tensor, segments, out: torch.Tensor, num_heads:
     tokens = min(qkv.shape[0], out.shape[0])
     if tokens == 0:
         return
-    flat = [int(x) for run in segments if run[1] and run[2] for x in run]
+    flat = [operator.index(x) for run in segments if run[1] and run[2] for x in run]
     triples = (ctypes.c_int64 * len(flat))(*flat)
     d, base, size = num_heads * ENCODER_HEAD_DIM, qkv.data_ptr(), qkv.element_size()
     check(lib.vfl_encoder_attention(
