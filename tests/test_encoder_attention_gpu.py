@@ -150,3 +150,11 @@ def test_empty_run_of_a_long_length():
     with torch.no_grad():
         layer.attend(qkv, [(0, 1, 30), (30, 0, 1000), (30, 1, 10)], out)
     check(out, qkv, [(0, 1, 30), (30, 1, 10)], 2)
+
+
+def test_autocast_type():
+    """Under autocast to another type the attention runs in that type, as torch's does."""
+    qkv = torch.randn(40, 384, device="cuda").to(torch.float16)
+    for dtype in (torch.float16, torch.bfloat16):
+        with torch.autocast("cuda", dtype=dtype):
+            assert hip_attn.encoder_attention_fits(qkv, None, 2, 0.125) == (dtype == qkv.dtype)

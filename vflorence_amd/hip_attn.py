@@ -733,6 +733,8 @@ def encoder_attention_fits(qkv: torch.Tensor, out: torch.Tensor | None, num_head
     if (not plain_eager() or not on_current_device(qkv)
             or (qkv.requires_grad and torch.is_grad_enabled())):
         return False
+    if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != qkv.dtype:
+        return False  # torch's attention runs in the autocast type
     if (qkv.stride(1) != 1 or qkv.stride(0) % 8 or qkv.stride(0) < qkv.shape[1]
             or qkv.data_ptr() % 16):
         return False
