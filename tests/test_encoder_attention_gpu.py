@@ -158,3 +158,24 @@ def test_autocast_type():
     for dtype in (torch.float16, torch.bfloat16):
         with torch.autocast("cuda", dtype=dtype):
             assert hip_attn.encoder_attention_fits(qkv, None, 2, 0.125) == (dtype == qkv.dtype)
+
+
+def test_in_place_rules():
+    """The write counts as one in place: a tensor saved for a gradient is known to have
+    changed, and an inference tensor is written in inference mode only."""
+    layer = BartEncoderSelfAttention(128, 2).cuda().to(torch.bfloat16)
+    qkv, runs = torch.randn(40, 384, device="cuda").to(torch.bfloat16), [(0, 1, 40)]
+    w = torch.ones(40, 128, dtype=qkv.dtype, device="cuda", requires_grad=True)
+    out = torch.zeros_like(qkv[:, :128])
+    y = (w * out).sum()
+    with torch.no_grad():
+        assert hip_attn.encoder_attention_fits(qkv, out, 2, 0.125)
+        layer.attend(qkv, runs, out)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.backward()
+    with torch.inference_mode():
+        out = torch.zeros_like(out)
+        layer.attend(qkv, runs, out)
+    check(out.clone(), qkv, runs, 2)
+    with torch.no_grad(), pytest.raises(RuntimeError, match="[Ii]nference"):
+        layer.attend(qkv, runs, out)

@@ -94,6 +94,6 @@ def test_runs_of_no_tokens(monkeypatch):
     runs = [(0, 2, 3), (6, 0, 1000), (6, 1, 4), (10, 0, 1 << 70), (10, 5, 0)]
     assert _runs_fit(runs, 10)
     hip_attn.encoder_attention(qkv, runs, out, 2, 0.125)
-    assert seen == [[0, 2, 3, 6, 1, 4]]
+    assert seen == [[0, 2, 3, 6, 1, 4]] and out._version == 1  # written in place
     with pytest.raises(TypeError):  # as a slice by it is
         hip_attn.encoder_attention(qkv, [(0, 1, 4.5)], out, 2, 0.125)

@@ -741,6 +741,7 @@ def encoder_attention_fits(qkv: torch.Tensor, out: torch.Tensor | None, num_head
     return out is None or (type(out) is torch.Tensor and out.device == qkv.device
                            and out.dtype == qkv.dtype and out.dim() == 2
                            and not out.requires_grad
+                           and (not out.is_inference() or torch.is_inference_mode_enabled())
                            and out.shape[1] == num_heads * ENCODER_HEAD_DIM
                            and out.stride(1) == 1 and out.stride(0) % 4 == 0
                            and out.stride(0) >= out.shape[1] and out.data_ptr() % 8 == 0
@@ -763,6 +764,7 @@ def encoder_attention(qkv: torch.Tensor, segments, out: torch.Tensor, num_heads:
         base, base + d * size, base + 2 * d * size, qkv.stride(0), out.data_ptr(), out.stride(0),
         tokens, triples, len(flat) // 3, num_heads, ENCODER_HEAD_DIM, float(scale),
         _dtype_code(qkv.dtype), _stream(qkv.device)))
+    torch.autograd.graph.increment_version(out)  # autograd's check of saved tensors
 
 
 def cache_pointer_table(caches: list[torch.Tensor]) -> torch.Tensor:
