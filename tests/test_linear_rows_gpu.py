@@ -60,3 +60,17 @@ def test_calls_that_stay_with_torch():
         torch.testing.assert_close(mapped[0], layer(x), rtol=2**-7, atol=2**-8)
         graph = torch.jit.trace(layer, x).graph
         assert "linear" in str(graph)
+
+
+@pytest.mark.parametrize("rows, out_f, in_f, kernel", [
+    (224, 2304, 768, True), (225, 2304, 768, False), (590, 2304, 768, False),
+    (672, 768, 768, True), (673, 768, 768, False), (1024, 768, 768, False),
+    (1024, 1024, 1024, True), (320, 3072, 1024, True), (321, 3072, 1024, False),
+    (455, 3072, 1024, False), (640, 1536, 512, True), (641, 1536, 512, False),
+    (1025, 64, 256, False),
+])
+def test_sizes_of_the_kernel(rows, out_f, in_f, kernel):
+    from vflorence_amd import decoder_ops as ops
+
+    x, w = (torch.empty(n, in_f, dtype=torch.bfloat16, device="cuda") for n in (rows, out_f))
+    assert ops.linear_rows_fits(x, w, None) == kernel

@@ -207,18 +207,25 @@ def _(x, packed_weight, bias, out_features, rows=-1, flags=0):
     return x.new_empty(*lead, out_features)
 
 
-# Where linear_rows takes an eager call, as rows and outputs (rows * out_features).  On the
-# device it is the faster one up to 1024 rows of a 768- or 1024-wide output (590 rows 6.4
-# against 7.6 us for hipBLASLt through torch, 1024 rows 9.2 against 9.4) and 250-400 rows of
-# a q|k|v (256 x 3072 9.2 against 9.3); above that the library call's 19 us of host time, to
-# 7 here, decide until the kernel takes as long (590 x 2304 13.2 us, 455 x 3072 15).
+# Where linear_rows takes a call: by time on the device alone, so that a caller whose GPU is
+# the one behind, or who records the call into a graph, loses nothing (where the host is
+# behind, torch's call costs 20 us of it and this one 11).  Rows padded to 32, times outputs;
+# against hipBLASLt through torch, both from graphs, in turn, 256 to 1024 inputs, us:
+# - up to 2^19, where the kernel's tiles of up to 64 x 32 take one round, it is the faster one:
+#   768 to 768 590 rows 6.5 / 7.5, 672 rows 6.6 / 7.4; 768 to 2304 224 rows 6.4 / 7.4; 1024 to
+#   1024 512 rows 7.1 / 8.6; 1024 to 3072 160 rows 7.1 / 8.5.
+# - up to 2^20, one round of 64 x 64 tiles, it is the faster one or level, but for 768 inputs:
+#   512 to 1536 640 rows 6.4 / 7.4; 1024 to 3072 320 rows 9.0 / 9.1; 1024 to 1024 1024 rows
+#   9.2 / 9.1; yet 768 to 768 704 rows 8.0 / 7.6, 768 to 2304 320 rows 7.9 / 7.7.
+# - beyond, the library: 768 to 2304 590 rows 13.3 / 9.4, 1024 to 3072 384 rows 13.0 / 10.1.
 LINEAR_ROWS_MAX = 1024
-LINEAR_ROWS_MAX_OUTPUTS = 1400000
+LINEAR_ROWS_MAX_OUTPUTS = 1 << 19
 
 
 def linear_rows_fits(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> bool:
-    """Whether ``linear_rows`` serves this call of nn.Linear: a plain eager call of 16-bit
-    tensors on the current GPU with rows aligned for its loads, nothing to differentiate."""
+    """Whether ``linear_rows`` serves this call of nn.Linear: of a size that it is the
+    faster one at, a plain eager (or captured) call of 16-bit tensors on the current GPU with
+    rows aligned for its loads, nothing to differentiate."""
     if not plain_eager() or torch.is_autocast_enabled(x.device.type):
         return False
     out_features, in_features = weight.shape
@@ -228,7 +235,8 @@ def linear_rows_fits(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor |
             and type(weight) in (torch.Tensor, torch.nn.Parameter)
             and x.shape[1] == in_features
             and 0 < x.shape[0] <= LINEAR_ROWS_MAX
-            and x.shape[0] * out_features <= LINEAR_ROWS_MAX_OUTPUTS
+            and ((x.shape[0] + 31) // 32 * 32 * out_features
+                 <= LINEAR_ROWS_MAX_OUTPUTS * (1 if in_features == 768 else 2))
             and out_features % 64 == 0 and in_features % LINEAR_K_MULTIPLE == 0
             and in_features <= 1024):
         return False

@@ -268,8 +268,8 @@ def _runs_fit(segments, rows: int) -> bool:
 
 
 class EncoderLinear(nn.Linear):
-    """nn.Linear whose small eager 16-bit calls run the split-K kernel on the weight as it
-    is (``decoder_ops.linear_rows``): there the library call is all host time."""
+    """nn.Linear whose small 16-bit calls, eager or captured, run the split-K kernel on the
+    weight as it is where that is the faster one (``decoder_ops.linear_rows_fits``)."""
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if x.is_cuda:
