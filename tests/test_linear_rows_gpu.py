@@ -66,7 +66,7 @@ def test_calls_that_stay_with_torch():
     (224, 2304, 768, True), (225, 2304, 768, False), (590, 2304, 768, False),
     (672, 768, 768, True), (673, 768, 768, False), (1024, 768, 768, False),
     (1024, 1024, 1024, True), (320, 3072, 1024, True), (321, 3072, 1024, False),
-    (455, 3072, 1024, False), (640, 1536, 512, True), (641, 1536, 512, False),
+    (455, 3072, 1024, False), (672, 1536, 512, True), (673, 1536, 512, False),
     (1025, 64, 256, False),
 ])
 def test_sizes_of_the_kernel(rows, out_f, in_f, kernel):
