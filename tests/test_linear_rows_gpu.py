@@ -74,3 +74,23 @@ def test_sizes_of_the_kernel(rows, out_f, in_f, kernel):
 
     x, w = (torch.empty(n, in_f, dtype=torch.bfloat16, device="cuda") for n in (rows, out_f))
     assert ops.linear_rows_fits(x, w, None) == kernel
+
+
+@pytest.mark.parametrize("shape", [(3, 45, 256), (2, 3, 7, 256), (1, 1, 256), (0, 4, 256)])
+def test_shapes_of_the_same_rows(shape):
+    """Equal tokens have equal bits in every shape of the call: prompts of equal length as
+    [prompts, tokens, d] and as packed rows."""
+    from vflorence_amd import decoder_ops as ops
+    from vflorence_amd.layers.bart import BartEncoderSelfAttention
+
+    g = torch.Generator(device="cuda").manual_seed(2)
+    layer = BartEncoderSelfAttention(256, 4).cuda().to(torch.bfloat16)
+    x, lin = rand(shape, g, torch.bfloat16), layer.out_proj
+    rows = x.view(-1, 256)
+    with torch.no_grad():
+        assert ops.linear_rows_fits(x, lin.weight, lin.bias) == bool(x.numel())
+        assert not ops.linear_rows_fits(x.transpose(0, 1), lin.weight, lin.bias) or shape[0] < 2
+        assert torch.equal(lin(x), lin(rows).view(shape))
+        if len(shape) == 3 and x.numel():
+            packed = layer(rows, [(0, *shape[:2])])
+            assert torch.equal(layer(x), packed.view(shape))

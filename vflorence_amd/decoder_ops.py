@@ -222,6 +222,16 @@ LINEAR_ROWS_MAX = 1024
 LINEAR_ROWS_MAX_OUTPUTS = 1 << 19
 
 
+def _rows_of(x: torch.Tensor) -> tuple[int, int] | None:
+    """Rows and row stride of ``x`` [..., in] taken as rows (more dimensions than two:
+    contiguous only), None where it is not."""
+    if x.dim() == 2 and x.stride(1) == 1:
+        return x.shape[0], x.stride(0)
+    if x.dim() > 2 and x.is_contiguous() and x.shape[-1]:
+        return x.numel() // x.shape[-1], x.shape[-1]
+    return None
+
+
 def linear_rows_fits(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> bool:
     """Whether ``linear_rows`` serves this call of nn.Linear: of a size that it is the
     faster one at, a plain eager (or captured) call of 16-bit tensors on the current GPU with
@@ -229,16 +239,20 @@ def linear_rows_fits(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor |
     if not plain_eager() or torch.is_autocast_enabled(x.device.type):
         return False
     out_features, in_features = weight.shape
-    if not (type(x) is torch.Tensor and x.is_cuda and on_current_device(x) and x.dim() == 2
+    if not (type(x) is torch.Tensor and x.is_cuda and on_current_device(x)
             and x.dtype in (torch.bfloat16, torch.float16)
             and weight.dtype == x.dtype and weight.device == x.device
             and type(weight) in (torch.Tensor, torch.nn.Parameter)
-            and x.shape[1] == in_features
-            and 0 < x.shape[0] <= LINEAR_ROWS_MAX
-            and ((x.shape[0] + 31) // 32 * 32 * out_features
-                 <= LINEAR_ROWS_MAX_OUTPUTS * (1 if in_features == 768 else 2))
             and out_features % 64 == 0 and in_features % LINEAR_K_MULTIPLE == 0
             and in_features <= 1024):
+        return False
+    at = _rows_of(x)
+    if at is None:
+        return False
+    rows, stride = at
+    if not (x.shape[-1] == in_features and 0 < rows <= LINEAR_ROWS_MAX
+            and ((rows + 31) // 32 * 32 * out_features
+                 <= LINEAR_ROWS_MAX_OUTPUTS * (1 if in_features == 768 else 2))):
         return False
     if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad
                                     or (bias is not None and bias.requires_grad)):
@@ -247,18 +261,17 @@ def linear_rows_fits(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor |
                                  and type(bias) in (torch.Tensor, torch.nn.Parameter)
                                  and bias.shape == (out_features,) and bias.is_contiguous()):
         return False
-    return (x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= in_features
-            and x.data_ptr() % 16 == 0 and weight.is_contiguous()
-            and weight.data_ptr() % 16 == 0)
+    return (stride % 8 == 0 and stride >= in_features and x.data_ptr() % 16 == 0
+            and weight.is_contiguous() and weight.data_ptr() % 16 == 0)
 
 
 def linear_rows(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
     """``x @ weight.T + bias`` for calls that ``linear_rows_fits`` accepts, from the weight's
     own layout (``vfl_linear_rows``)."""
-    rows, in_features = x.shape
-    out_features = weight.shape[0]
-    out = x.new_empty(rows, out_features)
-    check(lib.vfl_linear_rows(x.data_ptr(), x.stride(0), weight.data_ptr(),
+    rows, stride = _rows_of(x)
+    out_features, in_features = weight.shape
+    out = x.new_empty(*x.shape[:-1], out_features)
+    check(lib.vfl_linear_rows(x.data_ptr(), stride, weight.data_ptr(),
                               None if bias is None else bias.data_ptr(), out.data_ptr(),
                               out_features, rows, out_features, in_features,
                               _dtype_code(x.dtype), _stream(x.device)))
