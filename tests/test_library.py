@@ -323,3 +323,19 @@ def test_sched_meta_bindings_match_the_header(tmp_path):
         assert [getattr(binding, f).offset for f in names] == [o for _, o in c_fields]
         assert ctypes.sizeof(binding) == c_size
     assert "sizeof(SchedMeta) == 64" in _integration_sched_meta()[1]
+
+
+@pytest.mark.parametrize("bad", [
+    dict(dtype=0), dict(k=100), dict(k=1280), dict(n=80), dict(rows=65535 * 16 + 1), dict(rows=-1),
+    dict(ldx=255), dict(ldx=260), dict(ldy=63), dict(x=(1 << 20) + 8), dict(w=(1 << 21) + 8),
+    dict(y=(1 << 22) + 1), dict(bias=(1 << 23) + 1), dict(x=None), dict(w=None), dict(y=None),
+])
+def test_linear_rows_refused_calls(bad):
+    from vflorence_amd._lib import lib
+
+    def call(x=1 << 20, ldx=256, w=1 << 21, bias=1 << 23, y=1 << 22, ldy=64, rows=4, n=64, k=256,
+             dtype=1):
+        return lib.vfl_linear_rows(x, ldx, w, bias, y, ldy, rows, n, k, dtype, None)
+
+    assert call(**bad) < 0 and lib.vfl_last_error()
+    assert call(rows=0) == 0  # nothing to launch

@@ -51,7 +51,7 @@ def test_packed_layout_is_the_documented_operand_order():
     (1, 1024, 1024), (7, 1024, 1024), (64, 768, 768), (256, 1024, 1024), (256, 3072, 1024),
     (100, 1000, 512), (33, 1021, 256), (300, 96, 256), (5, 64, 4096), (40, 512, 1280),
     (17, 256, 2560), (256, 1024, 4096), (384, 3072, 1024), (512, 1024, 4096),
-    (448, 768, 768)])
+    (448, 768, 768), (16, 1280, 5120), (161, 5120, 1280)])
 @pytest.mark.parametrize("with_bias", [True, False])
 def test_linear_matches_float64(dtype, rows, out_f, in_f, with_bias):
     g = torch.Generator(device=DEV).manual_seed(rows * 7 + out_f)

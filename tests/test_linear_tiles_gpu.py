@@ -8,21 +8,24 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def rand(shape, g, scale=1.0):
-    return (torch.randn(*shape, device="cuda", generator=g) * scale).to(torch.bfloat16)
+def rand(shape, g, scale=1.0, dtype=torch.bfloat16):
+    return (torch.randn(*shape, device="cuda", generator=g) * scale).to(dtype)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("rows", [1, 15, 16, 17, 33, 129, 161, 193, 255, 257, 321, 385, 449, 512])
 @pytest.mark.parametrize("out_f,in_f", [(3072, 1024), (4096, 1024), (3072, 768), (2304, 768),
-                                        (1024, 1024), (768, 3072), (1024, 4096), (96, 2560)])
+                                        (1024, 1024), (768, 3072), (1024, 4096), (96, 2560),
+                                        (5120, 1280), (1280, 5120)])
 @pytest.mark.parametrize("step", [32, 16])
-def test_rows_do_not_depend_on_the_tile(rows, out_f, in_f, step):
+def test_rows_do_not_depend_on_the_tile(dtype, rows, out_f, in_f, step):
     from vflorence_amd import decoder_ops as ops
 
     g = torch.Generator(device="cuda").manual_seed(rows + out_f)
-    x, w = rand((rows, in_f), g), ops.pack_linear_weight(rand((out_f, in_f), g, in_f**-0.5))
-    bias, res = rand((out_f,), g), rand((rows, out_f), g)
-    gamma, beta = rand((out_f,), g), rand((out_f,), g)
+    x = rand((rows, in_f), g, dtype=dtype)
+    w = ops.pack_linear_weight(rand((out_f, in_f), g, in_f**-0.5, dtype))
+    bias, res = rand((out_f,), g, dtype=dtype), rand((rows, out_f), g, dtype=dtype)
+    gamma, beta = rand((out_f,), g, dtype=dtype), rand((out_f,), g, dtype=dtype)
     u, fb = (torch.randn(out_f, device="cuda", generator=g) for _ in range(2))
     x_stats = torch.rand(rows, in_f // 32, 2, device="cuda", generator=g)
     r_stats = torch.rand(rows, out_f // 32, 2, device="cuda", generator=g)
