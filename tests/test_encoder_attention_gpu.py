@@ -41,6 +41,9 @@ def check(out, qkv, segments, heads):
     (3, [(2, 31), (1, 32), (1, 33), (3, 64)]),       # edges of the query and key tiles
     (12, [(1, 590)]),                                # two key groups
     (1, [(1, 65)]), (2, [(1, 200)]),                 # as many key groups as key tiles; four
+    (2, [(1, 600)]),                                 # four key groups, three steps, the last ragged
+    (1, [(1, 1000), (1, 5), (2, 70)]),               # four, of which some see no key
+    (12, [(1, 590), (2, 20)]),                       # two, of which one sees no key
     (16, [(4, 129), (1, 127), (2, 128)]),            # two key groups
     (16, [(8, 1000), (0, 7), (5, 65), (3, 0)]),      # one key group; empty runs
     (2, [(1, 1 + 3 * i) for i in range(150)]),       # more runs than one launch holds
@@ -179,3 +182,67 @@ def test_in_place_rules():
     check(out.clone(), qkv, runs, 2)
     with torch.no_grad(), pytest.raises(RuntimeError, match="[Ii]nference"):
         layer.attend(qkv, runs, out)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("heads, length", [(1, 40), (2, 70), (2, 300), (12, 300), (16, 700)])
+def test_infinities_and_nan(dtype, heads, length):
+    """Infinite and NaN queries, keys and values come out where softmax attention has them,
+    and stay within their prompt and head; a query whose scores are all -inf is NaN."""
+    g = torch.Generator(device="cuda").manual_seed(length)
+    # weights far above the least 16-bit number, so that none is 0 against an infinite value
+    qkv = (torch.randn(6 * length, 3 * heads * 64, generator=g, device="cuda") / 2).to(dtype)
+    inf, nan, d = float("inf"), float("nan"), heads * 64
+    at = [slice(i * length, (i + 1) * length) for i in range(6)]
+    last = length - 1
+    qkv[at[0]][last, 2 * d + 3] = inf            # a value
+    qkv[at[1]][0, 2 * d + 5] = nan
+    qkv[at[2]][last, d + 1] = inf                # a key: scores of both signs
+    qkv[at[3]][1, 2] = nan                       # a query
+    qkv[at[4]][:, 0] = 1 + qkv[at[4]][:, 0].abs()
+    qkv[at[4]][:, d] = -inf                      # every score of the first head
+    segments = [(0, 6, length)]
+    out = torch.empty(6 * length, d, dtype=dtype, device="cuda")
+    assert hip_attn.encoder_attention_fits(qkv, out, heads, 0.125)
+    hip_attn.encoder_attention(qkv, segments, out, heads, 0.125)
+    ref, size = reference(qkv, segments, heads)
+    assert torch.equal(out.isnan(), ref.isnan()) and torch.equal(out.isinf(), ref.isinf())
+    assert torch.equal(out[ref.isinf()] > 0, ref[ref.isinf()] > 0)
+    assert bool(ref[at[4]][:, :64].isnan().all()) and bool(ref[at[5]].isfinite().all())
+    u = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-11  # the bound of check(), finite |v| <= 4
+    bound = 1.05 * u * (size + ref.abs()) + 2e-5 * size + length * 2.0**-25 * 4 + 1e-6
+    fine = ref.isfinite()
+    assert bool(((out.double() - ref).abs()[fine] <= bound[fine]).all())
+
+
+def test_replays_of_a_captured_launch():
+    g = torch.Generator(device="cuda").manual_seed(7)
+    layer = BartEncoderSelfAttention(256, 4).cuda().to(torch.bfloat16)
+    x, runs = torch.zeros(500, 256, dtype=torch.bfloat16, device="cuda"), [(0, 1, 300), (300, 4, 50)]
+    with torch.no_grad():
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            layer(x, runs)
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = layer(x, runs)
+        for _ in range(4):
+            x.copy_(torch.randn(500, 256, generator=g, device="cuda"))
+            want = layer(x, runs)
+            torch.cuda.synchronize()
+            graph.replay()
+            assert torch.equal(out, want)
+
+
+def test_runs_that_keep_torchs_path():
+    """Runs out of order, or that overlap, are taken in the order given."""
+    layer = BartEncoderSelfAttention(128, 2).cuda().to(torch.bfloat16)
+    qkv = torch.randn(90, 384, device="cuda").to(torch.bfloat16)
+    for runs in ([(30, 1, 60), (0, 2, 15)], [(0, 1, 50), (40, 1, 50)]):
+        out = torch.empty(90, 128, dtype=qkv.dtype, device="cuda")
+        with torch.no_grad():
+            assert hip_attn.encoder_attention_fits(qkv, out, 2, 0.125)
+            layer.attend(qkv, runs, out)
+        check(out, qkv, runs, 2)
