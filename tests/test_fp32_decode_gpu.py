@@ -1,6 +1,6 @@
-"""Decode attention over fp32 caches: the matrix-core kernel for row groups sharing a table
-and the fused K/V write, against 64-bit softmax attention of the same pages, at the edges
-of blocks, wave splits, group sizes and tables."""
+"""Decode attention over fp32 caches: row groups sharing a table, with and without slot
+descriptors, and the fused K/V write, both of the vector kernel, against 64-bit softmax
+attention of the same pages, at the edges of blocks, wave splits, group sizes and tables."""
 
 import pytest
 import torch

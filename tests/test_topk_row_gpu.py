@@ -42,6 +42,13 @@ def test_sizes_and_alignment(dtype, vocab, offset):
         check(logits, k, log_softmax, expect(logits, k, log_softmax))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_more_rows_than_compute_units(dtype):
+    g = torch.Generator(device="cuda").manual_seed(1)
+    logits = (torch.randn(513, 9001, device="cuda", generator=g) * 3).to(dtype)
+    check(logits, 8, True, expect(logits, 8, True))
+
+
 @pytest.mark.parametrize("tied", [3, 40, 200, 511, 513, 3000])
 def test_ties_at_the_threshold(tied):
     """``tied`` tokens share the second largest value: the lowest of them are listed."""
