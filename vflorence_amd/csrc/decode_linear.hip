@@ -11,8 +11,8 @@
 // trip per K step.  Here a workgroup owns an output tile (32 features x 32 tokens; others
 // by size, see pick_tile) and splits K over its 8 waves.  Each wave loads the operands of
 // up to 4 K steps of 32 in one batch, so K <= 1024 costs one round trip; a longer K range is
-// walked in batches of 2 steps with the next batch in flight while one is multiplied.  The
-// waves' partial tiles are summed through LDS in the order of a 3-level tree (waves w and
+// walked in batches of 2 steps with the next batch in flight while one is multiplied (a 32 x 16
+// tile: up to 16 steps in one batch, K <= 4096, then batches of 4).  The waves' partial tiles are summed through LDS in the order of a 3-level tree (waves w and
 // w + 4 first, then (s0 + s2) + (s1 + s3)), and the waves then add the bias and store a
 // 16 x 16 quarter each.
 //
@@ -293,9 +293,9 @@ __global__ __launch_bounds__(64 * LIN_WAVES) void decode_linear_kernel(
   static_assert(MODE != LIN_NORM_IN || !XP, "a pre-norm x is stored row by row");
   static_assert(!XP || TT <= 2, "packed activations are padded to 32 rows");
   constexpr int SUB = FT * TT;  // 16 x 16 quarters of the tile
-  // The 32 x 32 tile, of which a CU holds four, hands the partial tiles over in two halves
-  // (16 KB); the larger ones, one or two on a CU, all at once (64 or 128 KB, one barrier),
-  // and every wave finishes QPW quarters.
+  // The tiles up to 32 x 32 hand the partial tiles over in two halves (8 or 16 KB); the larger
+  // ones, one on a CU by their registers (157 to 256; 32 x 32: up to 124, two on a CU), all at
+  // once (64 or 128 KB, one barrier), and every wave finishes QPW quarters.
   constexpr bool HALVES = SUB < LIN_WAVES;
   constexpr int QPW = HALVES ? 1 : SUB / LIN_WAVES;
   static_assert(TT % QPW == 0, "a wave's quarters share their features");

@@ -6,7 +6,8 @@
 //   logprob_topk_kernel    -- per row: log-softmax of the logits, the generation rules
 //                             (min length, forced BOS / EOS, suppressed tokens), and the
 //                             k best (score, token) pairs, best first; one read of the
-//                             logits (logprob_topk_row_kernel), two for very long rows.  With log_softmax off the scores are the processed
+//                             logits (logprob_topk_row_kernel), two for very long rows.
+//                             With log_softmax off the scores are the processed
 //                             logits themselves (greedy decoding's argmax at k = 1).
 //
 // Both are bandwidth-bound streams over [rows, dim] / [rows, vocab] in HBM.
@@ -783,8 +784,10 @@ static int launch_topk(const void *logits, int64_t stride, int64_t rows, int voc
   using T = typename Elem<DT>::T;
   const dim3 grid((unsigned)rows);
   // One read wherever the row fits the workgroup's registers and the rules its short lists
-  // (k + bans must leave a bound among 64 group maxima, forced tokens one per lane): it
-  // was the faster one at every row count (4 to 256 rows: 7.5-8.9 against 19.7-21.0 us).
+  // (k + bans must leave a bound among 64 group maxima, forced tokens one per lane): it is the
+  // faster one at every row count, k and type (1 to 4096 rows x 50265, the k = 8 of 16-bit
+  // logits against the two-read kernel: 4 rows 7.6 / 19.8 us, 256 10.9 / 22.9, 512 18.1 / 30.6,
+  // 1024 32.0 / 49.1, 4096 119 / 153; fp32 512 rows 24.7 / 41.0, 4096 178 / 237).
   const int bans = rules.n_eos + rules.n_suppress + rules.n_begin;
   const int forced = rules.n_bos > rules.n_feos ? rules.n_bos : rules.n_feos;
   if (vocab <= TKR_VOCAB && bans <= TKR_LIST && forced <= TKR_LIST) {

@@ -3,9 +3,9 @@
 // launch, read from the fused q|k|v projection's rows and written to rows of the output
 // (vflorence/models/bart.py's encoder attention, SDPA there).
 //
-// What bounds it: the exponentials.  Per 32 queries x 64 keys a wave issues 16 matrix
-// products (512 cycles) and about 1000 cycles of vector work, half of it v_exp_f32; two or
-// more waves per SIMD overlap the two.
+// What bounds it: the vector work.  Per 32 queries x 64 keys a wave issues 20 matrix
+// products (8 for the scores, 8 with V, 4 that sum the weights: 640 cycles) and about 1000
+// cycles of vector work, half of it v_exp_f32; two or more waves per SIMD overlap the two.
 //
 // Tile.  Scores are computed transposed, S^T[key][query] = K Q^T (32x32x16 products), so a
 // lane holds one query's column: the softmax reduces inside the lane plus one half-wave
@@ -16,10 +16,13 @@
 // Precision: the weights are rounded to the element type for the second product, which
 // costs least where the running maximum is exact (the largest weight is 1, unrounded)
 // and the normalizer sums the rounded weights -- a third product, with a row of ones, which
-// also takes 32 additions per tile off the vector units.  Relative error against fp64,
-// bf16, 16 heads x 1024 keys: 1.82-1.83e-3 and SDPA 1.83-1.84e-3 (a reference that moves
-// only past a slack, as in the decode kernels: 2.09e-3 for 4% less time; weights split in
-// two 16-bit terms: 1.66e-3 for 25% more).
+// also takes 32 additions per tile off the vector units.  Error against fp64 (2-norm) over
+// that of SDPA, which sums the weights unrounded, 12 heads, 2 to 1024 keys, scores of standard
+// deviation 0.003 to 16: bf16 0.97-1.00 (flat 2.02e-3 both, 0.25 2.36e-3 / 2.36e-3, 1
+// 2.19e-3 / 2.22e-3, 4 1.70e-3 / 1.73e-3), fp16 0.96-1.00 (2.74e-4 / 2.78e-4 at 1); prompts of
+// two keys alone reach 1.003.  (A reference that moves only past a slack, as in the decode
+// kernels: 2.09e-3 against 1.83e-3 for 4% less time; weights split in two 16-bit terms:
+// 1.66e-3 for 25% more.)
 // K tiles sit in LDS row by row, 16-byte chunks xor-swizzled by the row against bank
 // conflicts; V tiles 4-key interleaved ([group][dim][4], transposed in registers on the
 // way in).  Tiles are double-buffered, the next one's loads in flight during the products.
