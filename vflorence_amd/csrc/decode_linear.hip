@@ -614,8 +614,12 @@ enum LinTile { TILE_32x16, TILE_32x32, TILE_64x32, TILE_64x64 };
 //   Elsewhere it is the slower one (1024 to 4096: 128 rows 8.1 / 10.4, 384 15.3 / 16.3).
 // - 64 x 32 where 32 x 32 tiles put a second workgroup on some CUs: 512 rows, 4096 to 1024
 //   15.8 / 13.4, 1024 to 1024 7.4 / 6.1; 128 rows, 768 to 3072 6.1 / 5.5, 1024 to 4096
-//   8.1 / 7.2.  With one on each it loses (256 rows, 1024 to 1024: 5.4 / 5.9).
-static LinTile pick_tile(int64_t rows, int out_features, bool packed_x, int mode) {
+//   8.1 / 7.2.  With one on each it loses (256 rows, 1024 to 1024: 5.4 / 5.9), and without
+//   row statistics (LIN_PLAIN) so it does up to 768 inputs, three K steps a wave: 512 rows, 768
+//   to 768 4.7 / 4.9 (352 rows 4.5 / 4.9); 128 rows, 768 to 2304 4.8 / 5.2; 320 rows, 512 to 1536
+//   4.2 / 4.4; yet 512 rows, 1024 to 1024 5.8 / 5.4.
+static LinTile pick_tile(int64_t rows, int out_features, int in_features, bool packed_x,
+                         int mode) {
   if (rows <= 16) return TILE_32x16;
   if (out_features % 64 != 0) return TILE_32x32;
   const int64_t t32 = out_features / 32 * ((rows + 31) / 32);
@@ -623,6 +627,7 @@ static LinTile pick_tile(int64_t rows, int out_features, bool packed_x, int mode
   if (!packed_x && mode != LIN_RESIDUAL &&
       ((t32 > 512 && t64 <= 256) || (t64 > 448 && t64 <= 512)))
     return TILE_64x64;
+  if (mode == LIN_PLAIN && in_features < LIN_BATCH * LIN_K_MULTIPLE) return TILE_32x32;
   return t32 > 256 && t32 <= 512 ? TILE_64x32 : TILE_32x32;
 }
 
@@ -633,7 +638,7 @@ static void launch_linear(hipStream_t s, int dtype, const void *x, int64_t x_str
                           const void *wp, const void *bias, void *y, int64_t y_stride,
                           int64_t rows, int out_features, int in_features, bool vec_store,
                           const LinNorm &nrm = LinNorm{}) {
-  const LinTile tile = pick_tile(rows, out_features, XP, MODE);
+  const LinTile tile = pick_tile(rows, out_features, in_features, XP, MODE);
   const int steps = in_features / LIN_K_MULTIPLE;
 #define VFL_TILE(P, FT, TT, B)                                                               \
   launch_linear_dt<XP, GELU, YP, P, MODE, FT, TT, B>(s, dtype, x, x_stride, wp, bias, y,     \
@@ -761,7 +766,7 @@ extern "C" int vfl_linear_rows(const void *x, int64_t x_stride, const void *weig
   launch_linear_dt<false, false, false, false, LIN_PLAIN, FT, TT, LIN_BATCH, true>(          \
       (hipStream_t)stream, dtype, x, x_stride, weight, bias, y, y_stride, rows, out_features, \
       in_features, vec_store, LinNorm{})
-  switch (pick_tile(rows, out_features, false, LIN_PLAIN)) {
+  switch (pick_tile(rows, out_features, in_features, false, LIN_PLAIN)) {
     case TILE_32x16: VFL_TILE(2, 1); break;
     case TILE_32x32: VFL_TILE(2, 2); break;
     case TILE_64x32: VFL_TILE(4, 2); break;

@@ -212,8 +212,8 @@ def _(x, packed_weight, bias, out_features, rows=-1, flags=0):
 # behind, torch's call costs 20 us of it and this one 11).  Rows padded to 32, times outputs;
 # against hipBLASLt through torch, both from graphs, in turn, 256 to 1024 inputs, us:
 # - up to 2^19, where the kernel's tiles of up to 64 x 32 take one round, it is the faster one:
-#   768 to 768 590 rows 6.5 / 7.5, 672 rows 6.6 / 7.4; 768 to 2304 224 rows 6.4 / 7.4; 1024 to
-#   1024 512 rows 7.1 / 8.6; 1024 to 3072 160 rows 7.1 / 8.5.
+#   768 to 768 590 rows 6.3 / 7.4, 672 rows 6.6 / 7.4; 768 to 2304 224 rows 6.0 / 7.4; 1024 to
+#   1024 512 rows 7.1 / 8.5; 1024 to 3072 160 rows 7.0 / 8.5.
 # - up to 2^20, one round of 64 x 64 tiles, it is the faster one or level, but for 768 inputs:
 #   512 to 1536 640 rows 6.4 / 7.4; 1024 to 3072 320 rows 9.0 / 9.1; 1024 to 1024 1024 rows
 #   9.2 / 9.1; yet 768 to 768 704 rows 8.0 / 7.6, 768 to 2304 320 rows 7.9 / 7.7.
