@@ -97,3 +97,25 @@ def test_runs_of_no_tokens(monkeypatch):
     assert seen == [[0, 2, 3, 6, 1, 4]] and out._version == 1  # written in place
     with pytest.raises(TypeError):  # as a slice by it is
         hip_attn.encoder_attention(qkv, [(0, 1, 4.5)], out, 2, 0.125)
+
+
+@pytest.mark.parametrize("dtype, count, length, kernel", [
+    (torch.bfloat16, 64, 16, True), (torch.bfloat16, 65, 16, False), (torch.bfloat16, 65, 17, True),
+    (torch.float16, 170, 1, True), (torch.float16, 171, 1, False), (torch.float16, 342, 17, False),
+    (torch.float16, 342, 33, True), (torch.bfloat16, 342, 17, True),
+])
+def test_many_short_prompts(monkeypatch, dtype, count, length, kernel):
+    """12 heads: one run of many short prompts keeps torch's path, two runs do not."""
+    seen = []
+    monkeypatch.setattr(hip_attn, "encoder_attention_fits", lambda *a: True)
+    monkeypatch.setattr(hip_attn, "encoder_attention", lambda *a: seen.append(a))
+    layer, rows = BartEncoderSelfAttention(768, 12).to(dtype), count * length
+    qkv, out = torch.zeros(rows + 1, 2304, dtype=dtype), torch.zeros(rows + 1, 768, dtype=dtype)
+    layer.attend(qkv, [(0, count, length), (rows, 0, 9)], out)
+    assert len(seen) == kernel
+    layer.attend(qkv, [(0, count, length), (rows, 1, 1)], out)
+    assert len(seen) == kernel + 1
+    if length == 1:
+        with torch.no_grad():
+            layer.attention(torch.zeros(count, length, 768, dtype=dtype))
+        assert len(seen) == 2 * kernel + 1

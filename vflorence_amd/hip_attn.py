@@ -748,6 +748,22 @@ def encoder_attention_fits(qkv: torch.Tensor, out: torch.Tensor | None, num_head
                            and not _spans_meet(qkv, out))
 
 
+def torch_attention_pays(segments, num_heads: int, dtype: torch.dtype) -> bool:
+    """Whether torch's attention is the faster one although ``encoder_attention`` serves the
+    call: one run of many prompts of up to 16 tokens, which a workgroup of 128 queries leaves
+    mostly empty.  Kernel against torch with the copy of its result, 12 heads, us: bf16, 64
+    prompts of 16 tokens 5.9 / 6.9, 75 7.8 / 7.4, 341 22.0 / 13.9; fp16 170 13.7 / 14.4, 341
+    23.2 / 22.6, and of up to 32 tokens 682 49.3 / 46.7 (24 tokens; bf16 level).  More runs
+    are a launch and a copy each for torch."""
+    runs = [run for run in segments if run[1] and run[2]]
+    if len(runs) != 1:
+        return False
+    pairs, length = runs[0][1] * num_heads, runs[0][2]
+    if length <= 16:
+        return pairs > (768 if dtype == torch.bfloat16 else 2048)
+    return length <= 32 and dtype == torch.float16 and pairs > 4096
+
+
 def encoder_attention(qkv: torch.Tensor, segments, out: torch.Tensor, num_heads: int,
                       scale: float) -> None:
     """Self-attention of packed prompts (``vfl_encoder_attention``): ``qkv`` ``[tokens, 3 d]``

@@ -298,9 +298,11 @@ class BartEncoderSelfAttention(_Heads):
             b, s, _ = x.shape
             qkv = self.qkv_proj(x)
             rows = qkv.reshape(b * s, 3 * self.embed_dim)
-            if hip_attn.encoder_attention_fits(rows, None, self.num_heads, self.scaling):
+            runs = ((0, b, s),)
+            if (hip_attn.encoder_attention_fits(rows, None, self.num_heads, self.scaling)
+                    and not hip_attn.torch_attention_pays(runs, self.num_heads, rows.dtype)):
                 out = rows.new_empty(b * s, self.embed_dim)
-                hip_attn.encoder_attention(rows, ((0, b, s),), out, self.num_heads, self.scaling)
+                hip_attn.encoder_attention(rows, runs, out, self.num_heads, self.scaling)
                 return out.view(b, s, self.embed_dim)
             q, k, v = (t.view(b, s, self.num_heads, self.head_dim).transpose(1, 2)
                        for t in qkv.chunk(3, dim=-1))
@@ -314,10 +316,12 @@ class BartEncoderSelfAttention(_Heads):
         """Attention of each run of equal-length prompts over the packed projections
         ``qkv`` [>= T, 3 d], written to rows ``start .. start + count * length`` of
         ``out``; other rows are left as they are.  One launch for all runs where the
-        packed kernel serves the call (hip_attn.encoder_attention_fits), else SDPA per run."""
+        packed kernel serves the call (hip_attn.encoder_attention_fits) and is the faster
+        one (hip_attn.torch_attention_pays), else SDPA per run."""
         segments = [tuple(run) for run in segments]  # read more than once below
         if (hip_attn.encoder_attention_fits(qkv, out, self.num_heads, self.scaling)
-                and _runs_fit(segments, min(qkv.shape[0], out.shape[0]))):
+                and _runs_fit(segments, min(qkv.shape[0], out.shape[0]))
+                and not hip_attn.torch_attention_pays(segments, self.num_heads, qkv.dtype)):
             hip_attn.encoder_attention(qkv, segments, out, self.num_heads, self.scaling)
             return
         for start, count, length in segments:
