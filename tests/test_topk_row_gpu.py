@@ -8,7 +8,8 @@ import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
-ROWS, LAST = 56 * 1024 - 16, 33  # vocabulary and rule list where the kernel hands over
+# vocabulary, forced and banned tokens where the kernel hands over
+ROWS, LAST, BANS = 56 * 1024 - 16, 33, 21
 
 
 def expect(logits, k, log_softmax, bans=(), forced=None):
@@ -43,9 +44,14 @@ def test_sizes_and_alignment(dtype, vocab, offset):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-def test_more_rows_than_compute_units(dtype):
-    g = torch.Generator(device="cuda").manual_seed(1)
-    logits = (torch.randn(513, 9001, device="cuda", generator=g) * 3).to(dtype)
+@pytest.mark.parametrize("rows, vocab", [
+    (3, 448), (3, 449), (3, 896), (3, 897),              # as many groups as k = 8 takes
+    (257, 704), (257, 705), (257, 1408), (257, 1409),    # half as many again
+    (512, 9001), (513, 9001), (513, 11999), (513, 12000), (513, 19999), (513, 20000),
+])
+def test_sizes_around_the_rule(dtype, rows, vocab):
+    g = torch.Generator(device="cuda").manual_seed(rows + vocab)
+    logits = (torch.randn(rows, vocab, device="cuda", generator=g) * 3).to(dtype)
     check(logits, 8, True, expect(logits, 8, True))
 
 
@@ -71,7 +77,7 @@ def test_rows_of_few_finite_values(finite):
         check(logits, 8, True, expect(logits, 8, True))
 
 
-@pytest.mark.parametrize("count", [1, 17, LAST - 1, LAST, 200])
+@pytest.mark.parametrize("count", [1, 17, BANS - 1, BANS, LAST - 1, LAST, 200])
 @pytest.mark.parametrize("k", [1, 16])
 def test_rule_lists(count, k):
     """Banned tokens that would be the best ones; forced tokens, some repeated, banned or
@@ -96,3 +102,10 @@ def test_rule_lists(count, k):
                                   device="cuda")
     lengths = torch.full((6,), 7, dtype=torch.int64, device="cuda")
     check(logits, k, True, expect(logits, k, True, bans=bans), lengths=lengths, rules=rules)
+    # forced tokens with one ban: the limits of the two lists are apart
+    rules = decoder_ops.TopkRules(eos=[2], suppress=[], begin_suppress=[forced[-1]], forced_bos=[],
+                                  forced_eos=forced, min_length=0, max_length=9, begin_index=8,
+                                  device="cuda")
+    lengths = torch.full((6,), 8, dtype=torch.int64, device="cuda")
+    check(logits, k, True, expect(logits, k, True, bans=forced[-1:], forced=forced),
+          lengths=lengths, rules=rules)

@@ -6,7 +6,8 @@
 //   logprob_topk_kernel    -- per row: log-softmax of the logits, the generation rules
 //                             (min length, forced BOS / EOS, suppressed tokens), and the
 //                             k best (score, token) pairs, best first; one read of the
-//                             logits (logprob_topk_row_kernel), two for very long rows.
+//                             logits (logprob_topk_row_kernel), two for very long rows,
+//                             short ones and long rule lists.
 //                             With log_softmax off the scores are the processed
 //                             logits themselves (greedy decoding's argmax at k = 1).
 //
@@ -418,8 +419,8 @@ __device__ __forceinline__ void topk_by_lists(const typename Elem<DT>::T *__rest
   }
 }
 
-// Row top-k in two reads of the row (the second mostly from L2), for rows and rule lists
-// that logprob_topk_row_kernel below does not take:
+// Row top-k in two reads of the row (the second mostly from L2), for what
+// logprob_topk_row_kernel below does not take (the rule is at launch_topk):
 //   1. each thread's largest allowed value, and the row maximum for the normaliser;
 //      the k-th largest of the per-thread maxima, tau, bounds the row's k-th value
 //      from below (k threads hold a value >= tau);
@@ -593,7 +594,8 @@ __global__ __launch_bounds__(NT, 2) void logprob_topk_kernel(
 // for the two-read kernel, 256 x 50265 8.9 against 21.0 (2.9 TB/s).
 constexpr int TKR_NT = 1024;
 constexpr int TKR_VOCAB = 56 * TKR_NT - 16;  // values a workgroup holds, less a scalar head
-constexpr int TKR_LIST = 32;  // longest rule list (banned, forced) that takes this kernel
+constexpr int TKR_LIST = 32;  // most forced tokens that take this kernel
+constexpr int TKR_BANS = 20;  // most banned tokens that do
 
 template <int DT, int K>
 __global__ __launch_bounds__(TKR_NT) void logprob_topk_row_kernel(
@@ -607,7 +609,7 @@ __global__ __launch_bounds__(TKR_NT) void logprob_topk_row_kernel(
   constexpr int CAP = 512;      // candidates kept in LDS
   constexpr int LPL = CAP / 64;
   static_assert(4 * NWAVE == 64, "one group maximum per lane");
-  __shared__ int s_ban[TKR_LIST];
+  __shared__ int s_ban[TKR_BANS];
   __shared__ int s_force[TKR_LIST];
   __shared__ float s_group[64];
   __shared__ float s_cv[CAP];
@@ -785,14 +787,33 @@ static int launch_topk(const void *logits, int64_t stride, int64_t rows, int voc
                        int log_softmax, int k, float *scores, int64_t *ids, hipStream_t stream) {
   using T = typename Elem<DT>::T;
   const dim3 grid((unsigned)rows);
-  // One read wherever the row fits the workgroup's registers and the rules its short lists
-  // (k + bans must leave a bound among 64 group maxima, forced tokens one per lane): it is the
-  // faster one at every row count, k and type (1 to 4096 rows x 50265, the k = 8 of 16-bit
-  // logits against the two-read kernel: 4 rows 7.6 / 19.8 us, 256 10.9 / 22.9, 512 18.1 / 30.6,
-  // 1024 32.0 / 49.1, 4096 119 / 153; fp32 512 rows 24.7 / 41.0, 4096 178 / 237).
+  // One read where the row fits the workgroup's registers and the rules its short lists
+  // (k + bans must leave a bound among 64 group maxima, forced tokens one per lane), and where
+  // that is the faster one.  Against the two-read kernel, us:
+  // - vocabularies of models and few bans, any row count: 50265 bf16 k = 8, 4 rows 7.6 / 19.8, 256
+  //   10.9 / 22.9, 512 18.1 / 30.6, 1024 32.0 / 49.1, 4096 119 / 153; fp32 512 rows 24.7 / 41.0,
+  //   4096 178 / 237.
+  // - a short row fills fewer groups than k + bans: no bound, and the whole row goes through
+  //   the lists (bf16 k = 16, 64 rows x 1500 31.1 / 22.2, x 2048 16.3 / 22.0).  With just as
+  //   many the bound is loose, which bans (64 x 3000, k = 1, 12 bans 12.6 / 14.0, 16 17.3 / 16.4) and
+  //   more rows than CUs (512 x 1000, k = 8 17.3 / 15.8, x 1500 13.7 / 16.0) feel.
+  // - bans move the bound down the 64 group maxima, and the candidates grow; the two-read
+  //   kernel has 512 (bf16, 256 rows x 13000, k = 8, 22 bans 25.5 / 27.9, 32 42.4 / 33.1; fp32, 512
+  //   rows x 50265, k = 16, 16 bans 45.2 / 59.2, 22 64.7 / 62.5; bf16, 512 x 3000, k = 1, 5 bans
+  //   11.7 / 11.4, 9 16.9 / 13.8).
+  // - of more than two rows per CU the two-read kernel's smaller workgroups get through more
+  //   short rows (640 rows, k = 8: bf16 x 3000 17.8 / 17.0, x 12000 18.0 / 18.9; fp32, 1024 rows x
+  //   12000 25.4 / 24.7, x 20000 29.6 / 33.1), but for k over 8, which its rounds of picks pay
+  //   for (640 rows x 4000, k = 16 20.0 / 26.9).
   const int bans = rules.n_eos + rules.n_suppress + rules.n_begin;
   const int forced = rules.n_bos > rules.n_feos ? rules.n_bos : rules.n_feos;
-  if (vocab <= TKR_VOCAB && bans <= TKR_LIST && forced <= TKR_LIST) {
+  constexpr int GROUP = 16 * 16 / (int)sizeof(T);  // values of a group's first vectors
+  const int groups = (vocab + GROUP - 1) / GROUP;
+  const bool bound = rows <= 256 ? groups >= k + bans + bans / 2 : 2 * groups >= 3 * (k + bans);
+  const bool few_bans = rows <= 256 || bans <= 1 + vocab / (rows <= 512 ? 3000 : 4000);
+  const bool long_rows = rows <= 512 || k > 8 || vocab >= (DT == VFL_FLOAT32 ? 20000 : 12000);
+  if (vocab <= TKR_VOCAB && bans <= TKR_BANS && forced <= TKR_LIST && bound && few_bans &&
+      long_rows) {
 #define VFL_TKR(KK)                                                                            \
   logprob_topk_row_kernel<DT, KK><<<grid, dim3(TKR_NT), 0, stream>>>(                          \
       (const T *)logits, stride, vocab, lengths, rule_tokens, rules, log_softmax, k, scores, ids)
