@@ -50,7 +50,7 @@ inline bool head_dim_native(int d) { return d == 64 || d == 128; }
 
 // fp32 caches: VALU kernel over the logical V layout, G query rows per group; pool
 // blocks of 16 << SHIFT tokens.
-template <int D, int G, int NW, int SHIFT = 0, bool FUSE = false>
+template <int D, int G, int NW, int SHIFT = 0, bool FUSE = false, bool DESC = false>
 int launch_valu(const AttnArgs &a) {
   constexpr int DT = VFL_FLOAT32;
   using T = typename Elem<DT>::T;
@@ -60,7 +60,7 @@ int launch_valu(const AttnArgs &a) {
                                (const T *)a.kvw.v, a.kvw.v_st, a.kvw.v_sh,
                                a.kvw.slots,        (T *)a.kc,  (T *)a.vc};
   paged_decode_kernel<DT, D, BS, G, NW, stage_blocks<DT, D, G>(), stage_pipeline<G>(), SHIFT,
-                      FUSE>
+                      FUSE, DESC>
       <<<grid, dim3(NW * 64), 0, a.stream>>>(
       (const T *)a.q, a.q_st, a.q_sh, (const T *)a.kc, (const T *)a.vc, (T *)a.out, a.seq_lens,
       a.bt, a.bt_stride, a.max_blocks, a.group_start, a.group_order, a.num_rows, a.num_groups,
@@ -68,19 +68,24 @@ int launch_valu(const AttnArgs &a) {
   return launch_status("attention_with_kv_cache");
 }
 
-template <int D, int G>
+template <int D, int G, bool DESC = false>
 int valu_waves(const AttnArgs &a, int nw) {
   switch (nw) {
-    case 1: return launch_valu<D, G, 1>(a);
-    case 2: return launch_valu<D, G, 2>(a);
-    case 4: return launch_valu<D, G, 4>(a);
-    default: return launch_valu<D, G, 8>(a);
+    case 1: return launch_valu<D, G, 1, 0, false, DESC>(a);
+    case 2: return launch_valu<D, G, 2, 0, false, DESC>(a);
+    case 4: return launch_valu<D, G, 4, 0, false, DESC>(a);
+    default: return launch_valu<D, G, 8, 0, false, DESC>(a);
   }
 }
 
 template <int D>
 int valu_group(const AttnArgs &a, int gmax, int nw) {
   if (gmax <= 1) return valu_waves<D, 1>(a, nw);
+  if (a.desc != nullptr) {
+    if (gmax <= 2) return valu_waves<D, 2, true>(a, nw);
+    if (gmax <= 4) return valu_waves<D, 4, true>(a, nw);
+    return valu_waves<D, 8, true>(a, nw);
+  }
   if (gmax <= 2) return valu_waves<D, 2>(a, nw);
   if (gmax <= 4) return valu_waves<D, 4>(a, nw);
   return valu_waves<D, 8>(a, nw);

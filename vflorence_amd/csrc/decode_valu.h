@@ -189,11 +189,15 @@ template <int DT> struct ValuKvWrite {
 // SHIFT: pool blocks hold BS << SHIFT tokens (0, or 1 for the reference's 32-token
 // blocks); the kernel walks BS-token parts of them.
 // FUSE (one row per workgroup): also writes the row's new token at its slot, under the
-// fused write's contract (see paged_decode_mfma_kernel, and desc there).  Where the slot is the row's last
+// fused write's contract (see paged_decode_mfma_kernel).  Where the slot is the row's last
 // position, the wave that reads that block puts the token into its registers and stores
 // it; a slot elsewhere is written by wave 0.  With a separate scatter launch the 64 rows
 // x 72 tokens of a layer took 4.8 + 9.4 us, fused 10.0.
-template <int DT, int D, int BS, int G, int NW, int U, bool PIPE, int SHIFT, bool FUSE>
+// DESC (row groups): the group comes from its slot descriptor (desc, as in
+// paged_decode_mfma_kernel).  A kernel of its own: chosen inside the launch it cost calls
+// without descriptors 1-2%, and at head size 512 twice the spilled registers (8 beams x 64
+// requests x 500 tokens 421 against 398 us).
+template <int DT, int D, int BS, int G, int NW, int U, bool PIPE, int SHIFT, bool FUSE, bool DESC>
 __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(
     const typename Elem<DT>::T *__restrict__ q, int64_t q_st, int64_t q_sh,
     const typename Elem<DT>::T *__restrict__ kc, const typename Elem<DT>::T *__restrict__ vc,
@@ -205,6 +209,7 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(
   using Lay = ValuLayout<DT, D>;
   constexpr int bs_shift = SHIFT;
   static_assert(!FUSE || (G == 1 && SHIFT == 0 && !PIPE), "the fused write is one row's");
+  static_assert(!DESC || (G > 1 && SHIFT == 0), "descriptors are of row groups");
   constexpr int VEC = Lay::VEC, CPL = Lay::CPL, LPT = Lay::LPT, TPL = Lay::TPL;
   constexpr int NLD = BS / TPL;  // loads per block per head and chunk slot
   static_assert(64 % LPT == 0 && BS % TPL == 0, "unsupported tile");
@@ -223,15 +228,13 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(
   if (pos >= num_groups || h >= H) return;
   int row0, nrows = 1, L;
   WaveBlockIds ids;
-  const bool described = G > 1 && SHIFT == 0 && desc != nullptr;
-  if (described) {
+  if constexpr (DESC) {
     const int32_t *rec = desc + pos * desc_stride;
     const int4 hdr = *reinterpret_cast<const int4 *>(rec);
     ids.prefetch(rec + 4, max_blocks);
     row0 = hdr.x;
     nrows = min(hdr.y, G);
     L = hdr.z;
-    if (row0 < 0 || row0 >= num_rows) return;
   } else {
     int g = (int)pos;
     if (group_order) g = group_order[g];
@@ -241,11 +244,11 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(
       row0 = group_start[g];
       nrows = min(group_start[g + 1] - row0, G);
     }
-    if (row0 < 0 || row0 >= num_rows) return;
-    L = seq_lens[row0];
   }
+  if (row0 < 0 || row0 >= num_rows) return;
   nrows = (int)min((int64_t)nrows, num_rows - row0);
   if (nrows <= 0) return;
+  if constexpr (!DESC) L = seq_lens[row0];
   int nblk = L > 0 ? (L + BS - 1) / BS : 0;  // BS-token chunks
   nblk = min(nblk, max_blocks << bs_shift);
   const int Lc = min(L, nblk * BS);
@@ -304,7 +307,7 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(
     for (int d = 0; d < CPL * VEC; ++d) acc[gi][d] = 0.f;
   }
 
-  if (described)
+  if constexpr (DESC)
     ids.limit(b1);
   else if constexpr (SHIFT == 0)
     ids.init(bt + (int64_t)row0 * bt_stride, b0, b1);
