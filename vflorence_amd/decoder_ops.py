@@ -236,15 +236,12 @@ def linear_rows_fits(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor |
     """Whether ``linear_rows`` serves this call of nn.Linear: of a size that it is the
     faster one at, a plain eager (or captured) call of 16-bit tensors on the current GPU with
     rows aligned for its loads, nothing to differentiate."""
-    if not plain_eager() or torch.is_autocast_enabled(x.device.type):
+    if not plain_eager() or type(x) is not torch.Tensor or not x.is_cuda:
         return False
+    dtype = x.dtype
     out_features, in_features = weight.shape
-    if not (type(x) is torch.Tensor and x.is_cuda and on_current_device(x)
-            and x.dtype in (torch.bfloat16, torch.float16)
-            and weight.dtype == x.dtype and weight.device == x.device
-            and type(weight) in (torch.Tensor, torch.nn.Parameter)
-            and out_features % 64 == 0 and in_features % LINEAR_K_MULTIPLE == 0
-            and in_features <= 1024):
+    if (dtype not in (torch.bfloat16, torch.float16) or in_features % LINEAR_K_MULTIPLE
+            or in_features > 1024 or out_features % 64):
         return False
     at = _rows_of(x)
     if at is None:
@@ -254,10 +251,16 @@ def linear_rows_fits(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor |
             and ((rows + 31) // 32 * 32 * out_features
                  <= LINEAR_ROWS_MAX_OUTPUTS * (1 if in_features == 768 else 2))):
         return False
+    if torch.is_autocast_enabled("cuda") or not on_current_device(x):
+        return False
+    device = x.device
+    if not (weight.dtype == dtype and weight.device == device
+            and type(weight) in (torch.Tensor, torch.nn.Parameter)):
+        return False
     if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad
                                     or (bias is not None and bias.requires_grad)):
         return False
-    if bias is not None and not (bias.dtype == x.dtype and bias.device == x.device
+    if bias is not None and not (bias.dtype == dtype and bias.device == device
                                  and type(bias) in (torch.Tensor, torch.nn.Parameter)
                                  and bias.shape == (out_features,) and bias.is_contiguous()):
         return False

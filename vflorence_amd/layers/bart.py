@@ -26,7 +26,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
-from .. import hip_attn
+from .. import decoder_ops, hip_attn
 from ..decoder_ops import LINEAR_MAX_IN, LINEAR_MAX_OUT, LINEAR_MAX_ROWS
 from .attention import decoder_cross_attention, decoder_self_attention
 
@@ -272,12 +272,10 @@ class EncoderLinear(nn.Linear):
     weight as it is where that is the faster one (``decoder_ops.linear_rows_fits``)."""
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        if x.is_cuda:
-            from .. import decoder_ops
-
-            if decoder_ops.linear_rows_fits(x, self.weight, self.bias):
-                return decoder_ops.linear_rows(x, self.weight, self.bias)
-        return super().forward(x)
+        weight, bias = self.weight, self.bias
+        if x.is_cuda and decoder_ops.linear_rows_fits(x, weight, bias):
+            return decoder_ops.linear_rows(x, weight, bias)
+        return F.linear(x, weight, bias)
 
 
 class BartEncoderSelfAttention(_Heads):
