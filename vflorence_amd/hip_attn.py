@@ -723,8 +723,9 @@ def encoder_attention_fits(qkv: torch.Tensor, out: torch.Tensor | None, num_head
                            scale: float) -> bool:
     """Whether ``encoder_attention`` serves these ``[tokens, 3 d]`` projections: 16-bit
     tensors of 64-wide heads on the current GPU whose rows are aligned for its loads, in a
-    plain eager call (nothing to differentiate, trace, batch or dispatch elsewhere), with an ``out`` that
-    shares no memory with them: a workgroup stores its rows while others still read."""
+    plain eager call (nothing to differentiate, trace, batch or dispatch elsewhere), with an
+    ``out`` that shares no memory with them: a workgroup stores its rows while others still
+    read."""
     if not (type(qkv) is torch.Tensor and qkv.is_cuda
             and qkv.dtype in (torch.bfloat16, torch.float16)
             and qkv.dim() == 2 and qkv.shape[1] == 3 * num_heads * ENCODER_HEAD_DIM
@@ -769,7 +770,8 @@ def encoder_attention(qkv: torch.Tensor, segments, out: torch.Tensor, num_heads:
     """Self-attention of packed prompts (``vfl_encoder_attention``): ``qkv`` ``[tokens, 3 d]``
     holds each token's q, k and v, ``segments`` lists ``(start, count, length)`` runs of
     equal-length prompts, and the rows they name of ``out`` ``[tokens, d]`` are written;
-    runs of no tokens are left out, whatever length they state.  For calls that ``encoder_attention_fits`` accepts."""
+    runs of no tokens are left out, whatever length they state.  For calls that
+    ``encoder_attention_fits`` accepts."""
     tokens = min(qkv.shape[0], out.shape[0])
     if tokens == 0:
         return
