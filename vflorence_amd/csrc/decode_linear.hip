@@ -12,9 +12,9 @@
 // by size, see pick_tile) and splits K over its 8 waves.  Each wave loads the operands of
 // up to 4 K steps of 32 in one batch, so K <= 1024 costs one round trip; a longer K range is
 // walked in batches of 2 steps with the next batch in flight while one is multiplied (a 32 x 16
-// tile: up to 16 steps in one batch, K <= 4096, then batches of 4).  The waves' partial tiles are summed through LDS in the order of a 3-level tree (waves w and
-// w + 4 first, then (s0 + s2) + (s1 + s3)), and the waves then add the bias and store a
-// 16 x 16 quarter each.
+// tile: up to 16 steps in one batch, K <= 4096, then batches of 4).  The waves' partial tiles
+// are summed through LDS in the order of a 3-level tree (waves w and w + 4 first, then (s0 +
+// s2) + (s1 + s3)), and the waves then add the bias and store a 16 x 16 quarter each.
 //
 // Operand order.  The product per 32-wide K step is mfma_f32_16x16x32 with A = 16
 // weight rows (features) and B = 16 token rows, giving D[feature][token]; a lane's four

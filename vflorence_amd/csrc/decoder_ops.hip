@@ -795,8 +795,8 @@ static int launch_topk(const void *logits, int64_t stride, int64_t rows, int voc
   //   4096 178 / 237.
   // - a short row fills fewer groups than k + bans: no bound, and the whole row goes through
   //   the lists (bf16 k = 16, 64 rows x 1500 31.1 / 22.2, x 2048 16.3 / 22.0).  With just as
-  //   many the bound is loose, which bans (64 x 3000, k = 1, 12 bans 12.6 / 14.0, 16 17.3 / 16.4) and
-  //   more rows than CUs (512 x 1000, k = 8 17.3 / 15.8, x 1500 13.7 / 16.0) feel.
+  //   many the bound is loose, which bans (64 x 3000, k = 1, 12 bans 12.6 / 14.0, 16 17.3 /
+  //   16.4) and more rows than CUs (512 x 1000, k = 8 17.3 / 15.8, x 1500 13.7 / 16.0) feel.
   // - bans move the bound down the 64 group maxima, and the candidates grow; the two-read
   //   kernel has 512 (bf16, 256 rows x 13000, k = 8, 22 bans 25.5 / 27.9, 32 42.4 / 33.1; fp32, 512
   //   rows x 50265, k = 16, 16 bans 45.2 / 59.2, 22 64.7 / 62.5; bf16, 512 x 3000, k = 1, 5 bans

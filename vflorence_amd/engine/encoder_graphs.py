@@ -8,8 +8,9 @@ part of the forward -- embeddings, projections, LayerNorms and feed-forward, the
 K/V projections and paging of every decoder layer -- is captured per token bucket (the
 step's tokens padded up to it): one graph before the first layer's attention, one
 between each layer's attention and the next, the last ending with the paging.  The
-attention of all prompts runs eagerly between them, over the real tokens only.  Padding tokens are row-wise values that nothing reads: attention leaves
-them out and their K/V slots are -1, which the slot write skips.
+attention of all prompts runs eagerly between them, over the real tokens only.  Padding
+tokens are row-wise values that nothing reads: attention leaves them out and their K/V
+slots are -1, which the slot write skips.
 """
 
 from __future__ import annotations
